@@ -57,21 +57,20 @@ __device__ __forceinline__ uint32_t from_f32_rne(float f) {
   }
 }
 
-// Eight fp32 values -> four packed 16-bit pairs (out[i] = v[2i] | v[2i+1] <<
-// 16), bit-identical to from_f32_rne on every element.  bf16: the hardware
+// 2 N fp32 values -> N packed 16-bit pairs (out[i] = v[2i] | v[2i+1] << 16),
+// bit-identical to from_f32_rne on every element.  bf16: the hardware
 // converter (v_cvt_pk_bf16_f32, round to nearest even, one instruction per
 // pair) gives the same bits for every non-NaN input; it would keep NaN
 // payload bits, so a lane holding a NaN redoes its packing with
 // from_f32_rne (0x7fc0).  fp16: from_f32_rne per element.
-template <bool BF16>
-__device__ __forceinline__ u32x4 pack8_rne(const float (&v)[8]) {
-  u32x4 out;
+template <bool BF16, int N>
+__device__ __forceinline__ void pack_rne(const float* v, uint32_t* out) {
   if constexpr (BF16) {
     typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
     typedef float f32x2 __attribute__((ext_vector_type(2)));
     bool nan = false;
 #pragma unroll
-    for (int i = 0; i < 4; ++i) {
+    for (int i = 0; i < N; ++i) {
       float a = v[2 * i], b = v[2 * i + 1];
       asm("" : "+v"(a));  // the rounded fp32 values, not a folded product
       asm("" : "+v"(b));
@@ -80,13 +79,26 @@ __device__ __forceinline__ u32x4 pack8_rne(const float (&v)[8]) {
     }
     if (nan) {
 #pragma unroll
-      for (int i = 0; i < 4; ++i) out[i] = from_f32_rne<true>(v[2 * i]) | (from_f32_rne<true>(v[2 * i + 1]) << 16);
+      for (int i = 0; i < N; ++i) out[i] = from_f32_rne<true>(v[2 * i]) | (from_f32_rne<true>(v[2 * i + 1]) << 16);
     }
   } else {
 #pragma unroll
-    for (int i = 0; i < 4; ++i) out[i] = from_f32_rne<false>(v[2 * i]) | (from_f32_rne<false>(v[2 * i + 1]) << 16);
+    for (int i = 0; i < N; ++i) out[i] = from_f32_rne<false>(v[2 * i]) | (from_f32_rne<false>(v[2 * i + 1]) << 16);
   }
-  return out;
+}
+
+template <bool BF16>
+__device__ __forceinline__ u32x4 pack8_rne(const float (&v)[8]) {
+  uint32_t w[4];
+  pack_rne<BF16, 4>(v, w);
+  return u32x4{w[0], w[1], w[2], w[3]};
+}
+
+template <bool BF16>
+__device__ __forceinline__ u32x2 pack4_rne(const float (&v)[4]) {
+  uint32_t w[2];
+  pack_rne<BF16, 2>(v, w);
+  return u32x2{w[0], w[1]};
 }
 
 // Two fp32 -> packed 16-bit pair using the hardware converter (RNE); used for

@@ -18,6 +18,8 @@
 //
 // This file is compiled with -ffp-contract=off; every fused multiply-add is
 // written out.
+#include <type_traits>
+
 #include "rope_math.hpp"
 
 namespace feattn {
@@ -32,40 +34,190 @@ constexpr int kDppHalfMirror = 0x141;   // lane i <- lane 7 - i within each 8-la
 constexpr int kDppQuadXor2 = 0x4e;      // quad_perm [2, 3, 0, 1]
 constexpr int kDppQuadXor1 = 0xb1;      // quad_perm [1, 0, 3, 2]
 
+constexpr int kDppRowRor8 = 0x128;      // lane ^ 8 within each 16-lane row
+
 // ---------------------------------------------------------------------------
-// fe_norm: one 256-thread block per row, any width.
+// fe_norm
 // ---------------------------------------------------------------------------
-template <bool BF16>
-__global__ __launch_bounds__(256) void norm_kernel(const uint16_t* __restrict__ x, const uint16_t* __restrict__ res,
-                                                   const uint16_t* __restrict__ w, uint16_t* __restrict__ out,
-                                                   uint16_t* __restrict__ new_res, int width, float eps) {
+// A stripe is 256 consecutive elements of a row: element t of stripe k is
+// term k of the tree's partial sum p[t].
+//
+// norm_row_kernel: one wavefront per row, the whole row in registers, read
+// once with 16-byte loads that are all issued before the first is used.  A
+// load instruction covers two stripes, lanes 0-31 the first and 32-63 the
+// second; one v_permlane32_swap per register pair then gives lane i four
+// consecutive elements of each of the two, t = 8c + 4 (i / 32) + 0..3 of its
+// chunk c, so that every p[t] is one lane's FMA chain.  Chunks go to lanes
+// in order, the upper four of each eight reversed: the tree's partner at
+// distance 32 is then the half-row mirror lane, and all its cross-lane steps
+// are register exchanges.  NP: stripe pairs a row may have (loads past the
+// row are redirected to its last elements and dropped).  HBM bound: 8192 x
+// 4096 bf16 with the residual takes 50.4 us, 5.3 TB/s of the 268 MB it needs
+// (a loop of 2-byte loads over the row, twice: 154 us; 8-byte loads without
+// the exchange: 53.7 us).
+__device__ __forceinline__ void swap_halves(uint32_t& a, uint32_t& b) {  // a's lanes 32-63 <-> b's lanes 0-31
+  const auto r = __builtin_amdgcn_permlane32_swap(a, b, false, false);
+  a = r[0];
+  b = r[1];
+}
+// Words 0, 1 become the lane's four elements of the first stripe of the pair,
+// words 2, 3 of the second; its own inverse.
+__device__ __forceinline__ u32x4 exchange_pair(u32x4 v) {
+  uint32_t a = v[0], b = v[2], c = v[1], d = v[3];
+  swap_halves(a, b);
+  swap_halves(c, d);
+  return u32x4{a, c, b, d};
+}
+
+template <bool BF16, int NP, bool RES, bool STREAM>
+__global__ __launch_bounds__(256) void norm_row_kernel(const uint16_t* x, const uint16_t* res,
+                                                       const uint16_t* __restrict__ w, uint16_t* out,
+                                                       uint16_t* new_res, int rows, int width, float eps) {
+  const int lane = threadIdx.x & 63;
+  const int row = blockIdx.x * (blockDim.x >> 6) + uniform(threadIdx.x >> 6);
+  if (row >= rows) return;
+  const int c8 = lane & 7;
+  const int j0 = 8 * ((lane & 56) | (c8 < 4 ? c8 : 11 - c8));
+  const size_t base = (size_t)row * width;
+  auto ld = [](const uint16_t* a) {
+    const u32x4* q = reinterpret_cast<const u32x4*>(a);
+    return STREAM ? __builtin_nontemporal_load(q) : *q;
+  };
+  auto put = [](uint16_t* a, u32x4 v) {
+    u32x4* q = reinterpret_cast<u32x4*>(a);
+    if constexpr (STREAM) __builtin_nontemporal_store(v, q);
+    else *q = v;
+  };
+  u32x4 xv[NP], rv[NP], wv[NP];
+#pragma unroll
+  for (int s = 0; s < NP; ++s) {
+    const int j = min(j0 + 512 * s, width - 8);
+    xv[s] = ld(x + base + j);
+    if constexpr (RES) rv[s] = ld(res + base + j);
+  }
+#pragma unroll
+  for (int s = 0; s < NP; ++s) wv[s] = *reinterpret_cast<const u32x4*>(w + min(j0 + 512 * s, width - 8));
+
+  float v[NP][8];
+  float p[4] = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+  for (int s = 0; s < NP; ++s) {
+    const bool in = j0 + 512 * s < width;
+    const u32x4 zero = {0u, 0u, 0u, 0u};  // elements that leave the chains as they are
+    const u32x4 xs = exchange_pair(in ? xv[s] : zero);
+    u32x4 rs = zero;
+    if constexpr (RES) rs = exchange_pair(in ? rv[s] : zero);
+#pragma unroll
+    for (int e = 0; e < 8; ++e) {
+      float a = (e & 1) ? hi_f32<BF16>(xs[e >> 1]) : lo_f32<BF16>(xs[e >> 1]);
+      if constexpr (RES) a = __fadd_rn(a, (e & 1) ? hi_f32<BF16>(rs[e >> 1]) : lo_f32<BF16>(rs[e >> 1]));
+      v[s][e] = a;
+      p[e & 3] = __builtin_fmaf(a, a, p[e & 3]);
+    }
+  }
+#pragma unroll
+  for (int e = 0; e < 4; ++e) p[e] = sum_x16(p[e]);                                  // step 128
+#pragma unroll
+  for (int e = 0; e < 4; ++e) p[e] = __fadd_rn(p[e], dpp<kDppRowRor8>(p[e]));        // step 64
+#pragma unroll
+  for (int e = 0; e < 4; ++e) p[e] = __fadd_rn(p[e], dpp<kDppHalfMirror>(p[e]));     // step 32
+#pragma unroll
+  for (int e = 0; e < 4; ++e) p[e] = __fadd_rn(p[e], dpp<kDppQuadXor2>(p[e]));       // step 16
+#pragma unroll
+  for (int e = 0; e < 4; ++e) p[e] = __fadd_rn(p[e], dpp<kDppQuadXor1>(p[e]));       // step 8
+#pragma unroll
+  for (int e = 0; e < 4; ++e) p[e] = sum_x32(p[e]);                                  // step 4
+  const float total = __fadd_rn(__fadd_rn(p[0], p[2]), __fadd_rn(p[1], p[3]));       // steps 2, 1
+  const float scale = rsqrt_rn(__fadd_rn(__fdiv_rn(total, (float)width), eps));
+#pragma unroll
+  for (int s = 0; s < NP; ++s) {
+    const int j = j0 + 512 * s;
+    const u32x4 ws = exchange_pair(wv[s]);
+    float o[8];
+#pragma unroll
+    for (int e = 0; e < 8; ++e)
+      o[e] = __fmul_rn(__fmul_rn(v[s][e], scale), (e & 1) ? hi_f32<BF16>(ws[e >> 1]) : lo_f32<BF16>(ws[e >> 1]));
+    const u32x4 ov = exchange_pair(pack8_rne<BF16>(o));
+    u32x4 nv;
+    if constexpr (RES) nv = exchange_pair(pack8_rne<BF16>(v[s]));
+    if (j < width) {
+      if constexpr (RES) {
+        if (new_res != nullptr) put(new_res + base + j, nv);
+      }
+      put(out + base + j, ov);
+    }
+  }
+}
+
+// norm_block_kernel: one 256-thread block per row, thread t walks p[t]'s
+// terms.  For few rows, where the latency of one row is the call's time and
+// four wavefronts get through it sooner than one, and for rows that
+// norm_row_kernel cannot read or hold.  The first KEEP stripes stay in
+// registers (their loads, and the weights', all in flight together); stripes
+// past them are read a second time.  64 rows of 4096: 4.0 us a call
+// (norm_row_kernel 5.4, a loop of dependent loads over the row 11.0); 4096
+// rows of 3001: 22.9 us against 50.4.
+template <bool BF16, int KEEP>
+__global__ __launch_bounds__(256) void norm_block_kernel(const uint16_t* x, const uint16_t* res,
+                                                       const uint16_t* __restrict__ w, uint16_t* out,
+                                                       uint16_t* new_res, int width, float eps) {
   __shared__ float part[256];
   const int t = threadIdx.x;
   const size_t base = (size_t)blockIdx.x * width;
-  float sum = 0.f;
-  for (int j = t; j < width; j += 256) {
+  auto load = [&](int j) {
     float v = to_f32<BF16>(x[base + j]);
     if (res != nullptr) v = __fadd_rn(v, to_f32<BF16>(res[base + j]));
-    sum = __builtin_fmaf(v, v, sum);
+    return v;
+  };
+  auto store = [&](int j, float v, float scale, uint32_t wj) {
+    if (new_res != nullptr) new_res[base + j] = (uint16_t)from_f32_rne<BF16>(v);
+    out[base + j] = (uint16_t)from_f32_rne<BF16>(__fmul_rn(__fmul_rn(v, scale), to_f32<BF16>(wj)));
+  };
+  uint32_t xr[KEEP], rr[KEEP], wr[KEEP];
+#pragma unroll
+  for (int k = 0; k < KEEP; ++k) xr[k] = x[base + min(t + 256 * k, width - 1)];
+  if (res != nullptr) {
+#pragma unroll
+    for (int k = 0; k < KEEP; ++k) rr[k] = res[base + min(t + 256 * k, width - 1)];
   }
+#pragma unroll
+  for (int k = 0; k < KEEP; ++k) wr[k] = w[min(t + 256 * k, width - 1)];
+  float v[KEEP];
+#pragma unroll
+  for (int k = 0; k < KEEP; ++k) v[k] = to_f32<BF16>(xr[k]);
+  if (res != nullptr) {
+#pragma unroll
+    for (int k = 0; k < KEEP; ++k) v[k] = __fadd_rn(v[k], to_f32<BF16>(rr[k]));
+  }
+  float sum = 0.f;
+#pragma unroll
+  for (int k = 0; k < KEEP; ++k) {
+    if (t + 256 * k >= width) v[k] = 0.f;  // leaves the chain as it is
+    sum = __builtin_fmaf(v[k], v[k], sum);
+  }
+  for (int j = t + 256 * KEEP; j < width; j += 256) {
+    const float y = load(j);
+    sum = __builtin_fmaf(y, y, sum);
+  }
+  // Every wavefront folds the 256 partial sums by itself (one barrier): two
+  // steps on what it reads, six in registers on the chunk order of
+  // norm_row_kernel.
   part[t] = sum;
   __syncthreads();
-  if (t < 128) part[t] = __fadd_rn(part[t], part[t + 128]);
-  __syncthreads();
-  if (t < 64) {
-    float s = __fadd_rn(part[t], part[t + 64]);
+  const int c8 = t & 7;
+  const int l = (t & 56) | (c8 < 4 ? c8 : 11 - c8);
+  float p = __fadd_rn(__fadd_rn(part[l], part[l + 128]), __fadd_rn(part[l + 64], part[l + 192]));  // steps 128, 64
+  p = sum_x32(p);                                // step 32
+  p = sum_x16(p);                                // step 16
+  p = __fadd_rn(p, dpp<kDppRowRor8>(p));         // step 8
+  p = __fadd_rn(p, dpp<kDppHalfMirror>(p));      // step 4
+  p = __fadd_rn(p, dpp<kDppQuadXor2>(p));        // step 2
+  p = __fadd_rn(p, dpp<kDppQuadXor1>(p));        // step 1
+  const float scale = rsqrt_rn(__fadd_rn(__fdiv_rn(p, (float)width), eps));
 #pragma unroll
-    for (int o = 32; o >= 1; o >>= 1) s = __fadd_rn(s, __shfl_xor(s, o, 64));
-    if (t == 0) part[0] = s;
-  }
-  __syncthreads();
-  const float scale = rsqrt_rn(__fadd_rn(__fdiv_rn(part[0], (float)width), eps));
-  for (int j = t; j < width; j += 256) {
-    float v = to_f32<BF16>(x[base + j]);
-    if (res != nullptr) v = __fadd_rn(v, to_f32<BF16>(res[base + j]));
-    if (new_res != nullptr) new_res[base + j] = (uint16_t)from_f32_rne<BF16>(v);
-    out[base + j] = (uint16_t)from_f32_rne<BF16>(__fmul_rn(__fmul_rn(v, scale), to_f32<BF16>(w[j])));
-  }
+  for (int k = 0; k < KEEP; ++k)
+    if (t + 256 * k < width) store(t + 256 * k, v[k], scale, wr[k]);
+  for (int j = t + 256 * KEEP; j < width; j += 256) store(j, load(j), scale, w[j]);
 }
 
 // ---------------------------------------------------------------------------
@@ -209,16 +361,61 @@ static int grid_for(int64_t work) {
   return (int)g;
 }
 
+template <bool BF16>
+static hipError_t norm_launch(const uint16_t* x, const uint16_t* res, const uint16_t* w, uint16_t* out,
+                              uint16_t* new_res, int rows, int width, float eps, hipStream_t st) {
+  const uintptr_t addr = (uintptr_t)x | (uintptr_t)res | (uintptr_t)w | (uintptr_t)out | (uintptr_t)new_res;
+  const int stripes = (width + 255) / 256;
+  // Up to two rows per compute unit: the block kernel (512 rows of 4096: 6.5
+  // against 8.2 us; 1024 rows: 10.1 against 8.8).
+  if (rows > 512 && width % 8 == 0 && addr % 16 == 0 && stripes <= 32 && (res != nullptr || new_res == nullptr)) {
+    // Two wavefronts per workgroup (8192 x 4096: 51.2 us, 52.5 with one, 52.7
+    // with four).
+    constexpr int wg = 2;
+    // Non-temporal accesses once a call no longer fits the XCDs' L2 (32 MiB):
+    // 33 MB 7.8 against 9.9 us without, 134 MB 26.3 against 27.6, 335 MB 62.1
+    // against 69.3; below, what the next kernel reads is left in L2 (a decode
+    // step's layers 151.2 us without the hint, 154.4 with).  Only where rows
+    // fill whole 128-byte lines: 8192 x 1000 takes 14.6 us with it, 11.0
+    // without.
+    const bool stream = width % 64 == 0 && (int64_t)rows * width * (res != nullptr ? 8 : 4) >= (int64_t(32) << 20);
+    auto go = [&](auto kernel) {
+      hipLaunchKernelGGL(kernel, dim3((rows + wg - 1) / wg), dim3(64 * wg), 0, st, x, res, w, out, new_res, rows,
+                         width, eps);
+    };
+    auto by_res = [&](auto np) {
+      constexpr int NP = decltype(np)::value;
+      if (res != nullptr) stream ? go(norm_row_kernel<BF16, NP, true, true>) : go(norm_row_kernel<BF16, NP, true, false>);
+      else stream ? go(norm_row_kernel<BF16, NP, false, true>) : go(norm_row_kernel<BF16, NP, false, false>);
+    };
+    if (stripes <= 2) by_res(std::integral_constant<int, 1>{});
+    else if (stripes <= 4) by_res(std::integral_constant<int, 2>{});
+    else if (stripes <= 8) by_res(std::integral_constant<int, 4>{});
+    else if (stripes <= 12) by_res(std::integral_constant<int, 6>{});
+    else if (stripes <= 16) by_res(std::integral_constant<int, 8>{});
+    else if (stripes <= 20) by_res(std::integral_constant<int, 10>{});
+    else if (stripes <= 24) by_res(std::integral_constant<int, 12>{});
+    else by_res(std::integral_constant<int, 16>{});
+    return hipGetLastError();
+  }
+  auto go = [&](auto kernel) {
+    hipLaunchKernelGGL(kernel, dim3(rows), dim3(256), 0, st, x, res, w, out, new_res, width, eps);
+  };
+  if (stripes <= 4) go(norm_block_kernel<BF16, 4>);
+  else if (stripes <= 8) go(norm_block_kernel<BF16, 8>);
+  else if (stripes <= 16) go(norm_block_kernel<BF16, 16>);
+  else go(norm_block_kernel<BF16, 24>);
+  return hipGetLastError();
+}
+
 hipError_t launch_norm(const void* x, const void* res, const void* w, void* out, void* new_res, int rows, int width,
                        float eps, bool bf16, hipStream_t st) {
   if (rows == 0) return hipSuccess;
-  if (bf16)
-    hipLaunchKernelGGL(norm_kernel<true>, dim3(rows), dim3(256), 0, st, (const uint16_t*)x, (const uint16_t*)res,
-                       (const uint16_t*)w, (uint16_t*)out, (uint16_t*)new_res, width, eps);
-  else
-    hipLaunchKernelGGL(norm_kernel<false>, dim3(rows), dim3(256), 0, st, (const uint16_t*)x, (const uint16_t*)res,
-                       (const uint16_t*)w, (uint16_t*)out, (uint16_t*)new_res, width, eps);
-  return hipGetLastError();
+  auto go = [&](auto bf) {
+    return norm_launch<decltype(bf)::value>((const uint16_t*)x, (const uint16_t*)res, (const uint16_t*)w,
+                                            (uint16_t*)out, (uint16_t*)new_res, rows, width, eps, st);
+  };
+  return bf16 ? go(std::true_type{}) : go(std::false_type{});
 }
 
 hipError_t launch_norm_rope_append(const void* qkv, int64_t row_stride, const void* qw, const void* kw, float eps,

@@ -50,6 +50,76 @@ def test_norm_bit_exact(dev, bf16, width, residual):
     assert np.array_equal(u16(xd), want)
 
 
+@pytest.mark.parametrize("bf16", [True, False])
+@pytest.mark.parametrize("width,offset", [(8, 0), (248, 0), (256, 0), (264, 0), (504, 0), (520, 0), (1024, 0),
+                                          (1032, 0), (3064, 0), (6144, 0), (8192, 0), (8200, 0), (1, 0), (257, 0),
+                                          (1022, 0), (3001, 0), (6145, 0), (512, 1), (4096, 4)])
+def test_norm_widths_and_alignments(dev, bf16, width, offset):
+    """Bit-exact on both sides of every stripe, pair and register bound of the
+    kernels, on widths that are no multiple of a load and on tensors that
+    start `offset` elements past an aligned address; guard elements stay.  5
+    rows take the block kernel, 515 (the same ones again and again) the
+    wavefront-per-row kernel wherever it applies."""
+    dt = dtype_of(bf16)
+    gen = torch.Generator().manual_seed(3 * width + offset)
+    rows, n, reps = 5, 5 * width, 103
+    x = (torch.randn(rows, width, generator=gen) * 3).to(dt)
+    r = torch.randn(rows, width, generator=gen).to(dt)
+    w = (1 + 0.1 * torch.randn(width, generator=gen)).to(dt)
+
+    def place(t):
+        buf = torch.full((offset + t.numel() + 8,), 7.0, dtype=dt, device=dev)
+        buf[offset:offset + t.numel()] = t.reshape(-1).to(dev)
+        return buf, buf[offset:]
+
+    for res in (None, r):
+        want, want_res = N.rms_norm(u16(x), u16(w), 1e-6, bf16, residual=None if res is None else u16(res))
+        (_, xd), (_, wd) = place(x), place(w)
+        rd = None if res is None else place(res)[1]
+        ob, out = place(torch.zeros(n))
+        nb, new_res = place(torch.zeros(n))
+        feattn.norm(xd, wd, out, rows, width, 1e-6, bf16, residual=rd, new_residual=new_res)
+        torch.cuda.synchronize()
+        assert np.array_equal(u16(out[:n]).reshape(rows, width), want)
+        assert np.array_equal(u16(new_res[:n]).reshape(rows, width), want_res if res is not None else u16(x))
+        for buf in (ob, nb):
+            assert (buf[:offset] == 7.0).all() and (buf[offset + n:] == 7.0).all()
+        many = rows * reps
+        (_, xd) = place(x.repeat(reps, 1))
+        rd = None if res is None else place(res.repeat(reps, 1))[1]
+        ob, out = place(torch.zeros(n * reps))
+        nb, new_res = place(torch.zeros(n * reps))
+        feattn.norm(xd, wd, out, many, width, 1e-6, bf16, residual=rd, new_residual=None if res is None else new_res)
+        torch.cuda.synchronize()
+        got = u16(out[:n * reps]).reshape(reps, rows, width)
+        assert np.array_equal(got, np.broadcast_to(want, got.shape))
+        if res is not None:
+            got = u16(new_res[:n * reps]).reshape(reps, rows, width)
+            assert np.array_equal(got, np.broadcast_to(want_res, got.shape))
+        for buf in (ob, nb):
+            assert (buf[:offset] == 7.0).all() and (buf[offset + n * reps:] == 7.0).all()
+
+
+@pytest.mark.parametrize("bf16", [True, False])
+def test_norm_large_call_equals_small_calls(dev, bf16):
+    """A call past the L2's size streams its tensors; every row's bits are
+    those of the same rows in small calls (the last one, of an odd count)."""
+    rows, width = 2051, 2048
+    gen = torch.Generator(device=dev).manual_seed(5)
+    x = (torch.randn(rows, width, generator=gen, device=dev) * 3).to(dtype_of(bf16))
+    r = torch.randn(rows, width, generator=gen, device=dev).to(x.dtype)
+    w = (1 + 0.1 * torch.randn(width, generator=gen, device=dev)).to(x.dtype)
+    out, new = torch.empty_like(x), torch.empty_like(x)
+    feattn.norm(x, w, out, rows, width, 1e-6, bf16, residual=r, new_residual=new)
+    part, part_new = torch.empty_like(x), torch.empty_like(x)
+    for i in range(0, rows, 300):
+        n = min(300, rows - i)
+        feattn.norm(x[i:], w, part[i:], n, width, 1e-6, bf16, residual=r[i:], new_residual=part_new[i:])
+    torch.cuda.synchronize()
+    assert torch.equal(out.view(torch.int16), part.view(torch.int16))
+    assert torch.equal(new.view(torch.int16), part_new.view(torch.int16))
+
+
 def make_fused_case(bf16, rows, hq, hkv, row_stride, seed, cache_pages=64, max_pos=4096):
     dt = dtype_of(bf16)
     gen = torch.Generator().manual_seed(seed)
