@@ -289,3 +289,58 @@ def test_silu_mul_within_one_step(dev, bf16):
     step = np.maximum(np.abs(a), np.abs(b)) * (2.0 ** -7 if bf16 else 2.0 ** -10) + (0 if bf16 else 2.0 ** -24)
     assert (np.abs(a - b) <= step).all()
     assert np.mean(got == want) > 0.99
+
+
+def silu_close(got, want, bf16):
+    """One rounding step of the 16-bit type; NaN for NaN, infinities and the
+    sign of results that underflow equal."""
+    a, b = R.to_f32(got, bf16).astype(np.float64), R.to_f32(want, bf16).astype(np.float64)
+    assert np.array_equal(np.isnan(a), np.isnan(b))
+    if bf16:
+        assert (got[np.isnan(a)] == 0x7FC0).all()
+    inf = np.isinf(a) | np.isinf(b)
+    assert np.array_equal(a[inf], b[inf])
+    ok = ~(np.isnan(a) | inf)
+    # a result below 2^-126 has float32's own absolute spacing behind it
+    step = np.maximum(np.abs(a), np.abs(b))[ok] * (2.0 ** -7 if bf16 else 2.0 ** -10) + (2.0 ** -133 if bf16
+                                                                                        else 2.0 ** -24)
+    assert (np.abs(a[ok] - b[ok]) <= step).all()
+
+
+@pytest.mark.parametrize("bf16", [True, False])
+@pytest.mark.parametrize("width,offset", [(65536, 0), (65536, 1), (8, 0), (24, 0), (1, 0), (1001, 0), (2056, 8)])
+def test_silu_mul_all_gates(dev, bf16, width, offset):
+    """Every 16-bit gate (NaNs, infinities, subnormals, both ends of the
+    exponential) in rows of widths around the vector kernel's chunk, and on
+    tensors `offset` elements past an aligned address."""
+    dt = dtype_of(bf16)
+    rows = max(1, 65536 // width)
+    gen = torch.Generator().manual_seed(width + offset)
+    x = torch.randperm(65536, generator=gen)[:rows * width].to(torch.int32).to(torch.int16).view(dt)
+    if width == 1:
+        x = torch.arange(65536, dtype=torch.int32).to(torch.int16).view(dt)
+    up = torch.randn(rows, width, generator=gen).to(dt)
+    gu = torch.cat([x.reshape(rows, width), up], 1)
+    with np.errstate(all="ignore"):
+        want = N.silu_mul(u16(gu), bf16)
+    buf = torch.zeros(offset + gu.numel(), dtype=dt, device=dev)
+    buf[offset:] = gu.reshape(-1).to(dev)
+    ob = torch.full((offset + rows * width + 8,), 7.0, dtype=dt, device=dev)
+    feattn.silu_mul(buf[offset:], ob[offset:], rows, width, bf16)
+    torch.cuda.synchronize()
+    silu_close(u16(ob[offset:offset + rows * width]).reshape(rows, width), want, bf16)
+    assert (ob[:offset] == 7.0).all() and (ob[offset + rows * width:] == 7.0).all()
+
+
+def test_silu_mul_large_call_equals_small_calls(dev):
+    """A call past the L2's size streams its tensors: the bits of the same
+    rows in small calls."""
+    rows, width = 1031, 6144
+    gen = torch.Generator(device=dev).manual_seed(9)
+    gu = (torch.randn(rows, 2 * width, generator=gen, device=dev) * 4).bfloat16()
+    out, part = (torch.empty(rows, width, device=dev, dtype=torch.bfloat16) for _ in range(2))
+    feattn.silu_mul(gu, out, rows, width, True)
+    for i in range(0, rows, 100):
+        feattn.silu_mul(gu[i:], part[i:], min(100, rows - i), width, True)
+    torch.cuda.synchronize()
+    assert torch.equal(out.view(torch.int16), part.view(torch.int16))
