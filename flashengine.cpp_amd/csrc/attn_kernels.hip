@@ -25,6 +25,7 @@
 #include <atomic>
 #include <type_traits>
 
+#include "attn_short.hpp"
 #include "attn_types.hpp"
 #include "device_util.hpp"
 #include "kernel_util.hpp"
@@ -92,14 +93,17 @@ __device__ __forceinline__ ShareStart ldc_share(const ShareStart* shares, int i)
   r.first = DecodeItem{v[2], v[3], v[4], v[5], v[6], v[7], v[8], v[9]};
   r.pg0 = v[10];
   r.pg1 = v[11];
+  r.n_short = v[12];
   return r;
 }
 
 // NCB: 16-column blocks per item (1 or 2: up to 32 (query row, head)
 // columns, e.g. 8 verify rows with 4 heads per kv head).  Four blocks would
 // need more than the 256 registers of two wavefronts per SIMD.
-template <bool BF16, int WAVES, int NCB>
-__global__ __launch_bounds__(64 * WAVES) void attn_decode_kernel(AttnArgs a, int causal) {
+// ANY: the launch of a graph plan, whose later prepares may plan the batch
+// as short-context items instead (short_items).
+template <bool BF16, int WAVES, int NCB, bool ANY>
+__global__ __launch_bounds__(64 * WAVES, ANY ? 2 : 1) void attn_decode_kernel(AttnArgs a, int causal) {
   constexpr int U = dec_units<WAVES>();
   static_assert(U >= 2, "the ring must hold one K/V pair");
   extern __shared__ __attribute__((aligned(16))) uint8_t dsm[];
@@ -119,8 +123,15 @@ __global__ __launch_bounds__(64 * WAVES) void attn_decode_kernel(AttnArgs a, int
   const int slot = blockIdx.x * WAVES + wave;
   const int kvh = slot % a.hkv;
   const int share = slot / a.hkv;
-  if (share >= a.n_share_cap) return;
-  const ShareStart rec = ldc_share(a.shares, share);
+  if (!ANY && share >= a.n_share_cap) return;
+  const ShareStart rec = ldc_share(a.shares, ANY ? min(share, a.n_share_cap - 1) : share);
+  if constexpr (ANY) {
+    if (rec.n_short > 0) {
+      short_items<BF16, WAVES, NCB>(a, causal, rec.n_short, dsm);
+      return;
+    }
+    if (share >= a.n_share_cap) return;
+  }
   const int it_begin = rec.it_begin;
   const int it_end = rec.it_end;
   if (it_begin >= it_end) return;
@@ -797,38 +808,68 @@ int decode_wg_waves(int hkv) {
 }
 
 template <bool BF16, int WAVES, int NCB>
+__global__ __launch_bounds__(64 * WAVES, 2) void attn_short_kernel(AttnArgs a, int causal) {
+  extern __shared__ __attribute__((aligned(16))) uint8_t dsm[];
+  short_items<BF16, WAVES, NCB>(a, causal, a.n_short, dsm);
+}
+
+enum class DecodeKind { Shares, Short, Any };
+
+template <bool BF16, int WAVES, int NCB, DecodeKind KIND>
 static hipError_t decode_launch(const AttnArgs& a, int causal, int grid, hipStream_t st) {
-  const size_t lds = (size_t)WAVES * dec_units<WAVES>() * kDecUnit + 16;
+  void (*fn)(AttnArgs, int);
+  size_t lds = 0;
+  if constexpr (KIND != DecodeKind::Short) lds = (size_t)WAVES * dec_units<WAVES>() * kDecUnit + 16;
+  if constexpr (KIND != DecodeKind::Shares) lds = std::max(lds, short_lds<WAVES>());
+  if constexpr (KIND == DecodeKind::Short) fn = attn_short_kernel<BF16, WAVES, NCB>;
+  else fn = attn_decode_kernel<BF16, WAVES, NCB, KIND == DecodeKind::Any>;
   static std::atomic<uint64_t> lds_ok{0};
-  const hipError_t e = allow_lds((const void*)attn_decode_kernel<BF16, WAVES, NCB>, lds, lds_ok);
+  const hipError_t e = allow_lds((const void*)fn, lds, lds_ok);
   if (e != hipSuccess) return e;
-  hipLaunchKernelGGL((attn_decode_kernel<BF16, WAVES, NCB>), dim3(grid), dim3(64 * WAVES), lds, st, a, causal);
+  hipLaunchKernelGGL(fn, dim3(grid), dim3(64 * WAVES), lds, st, a, causal);
   return hipGetLastError();
 }
 
-template <bool BF16, int WAVES>
+template <bool BF16, int WAVES, DecodeKind KIND>
 static hipError_t decode_launch_ncb(const AttnArgs& a, int ncb, int causal, int grid, hipStream_t st) {
   switch (ncb) {
-    case 1: return decode_launch<BF16, WAVES, 1>(a, causal, grid, st);
-    case 2: return decode_launch<BF16, WAVES, 2>(a, causal, grid, st);
+    case 1: return decode_launch<BF16, WAVES, 1, KIND>(a, causal, grid, st);
+    case 2: return decode_launch<BF16, WAVES, 2, KIND>(a, causal, grid, st);
     default: return hipErrorInvalidValue;
   }
+}
+
+// Workgroups of fewer than kShortMinWaves wavefronts have no short-context
+// form (the planner makes no such items for them).
+template <bool BF16, int WAVES>
+static hipError_t decode_launch_kind(const AttnArgs& a, int ncb, int causal, bool any, int grid, hipStream_t st) {
+  if constexpr (WAVES >= kShortMinWaves) {
+    if (any) return decode_launch_ncb<BF16, WAVES, DecodeKind::Any>(a, ncb, causal, grid, st);
+    if (a.n_short > 0) return decode_launch_ncb<BF16, WAVES, DecodeKind::Short>(a, ncb, causal, grid, st);
+  } else if (a.n_short > 0) {
+    return hipErrorInvalidValue;
+  }
+  return decode_launch_ncb<BF16, WAVES, DecodeKind::Shares>(a, ncb, causal, grid, st);
 }
 
 template <bool BF16>
-static hipError_t decode_launch_waves(const AttnArgs& a, int waves, int ncb, int causal, int grid, hipStream_t st) {
+static hipError_t decode_launch_waves(const AttnArgs& a, int waves, int ncb, int causal, bool any, int grid,
+                                      hipStream_t st) {
   switch (waves) {
-    case 8: return decode_launch_ncb<BF16, 8>(a, ncb, causal, grid, st);
-    case 4: return decode_launch_ncb<BF16, 4>(a, ncb, causal, grid, st);
-    case 2: return decode_launch_ncb<BF16, 2>(a, ncb, causal, grid, st);
-    case 1: return decode_launch_ncb<BF16, 1>(a, ncb, causal, grid, st);
+    case 8: return decode_launch_kind<BF16, 8>(a, ncb, causal, any, grid, st);
+    case 4: return decode_launch_kind<BF16, 4>(a, ncb, causal, any, grid, st);
+    case 2: return decode_launch_kind<BF16, 2>(a, ncb, causal, any, grid, st);
+    case 1: return decode_launch_kind<BF16, 1>(a, ncb, causal, any, grid, st);
     default: return hipErrorInvalidValue;
   }
 }
 
-hipError_t launch_decode(const AttnArgs& a, bool bf16, int waves, int ncb, int causal, int grid, hipStream_t st) {
-  return bf16 ? decode_launch_waves<true>(a, waves, ncb, causal, grid, st)
-              : decode_launch_waves<false>(a, waves, ncb, causal, grid, st);
+// any: a graph plan's launch, which takes whichever form the plan's latest
+// prepare chose; else a.n_short > 0 selects the short-context kernel.
+hipError_t launch_decode(const AttnArgs& a, bool bf16, int waves, int ncb, int causal, bool any, int grid,
+                         hipStream_t st) {
+  return bf16 ? decode_launch_waves<true>(a, waves, ncb, causal, any, grid, st)
+              : decode_launch_waves<false>(a, waves, ncb, causal, any, grid, st);
 }
 
 // Plan staging: copies a prepared metadata image from pinned host memory

@@ -15,6 +15,7 @@ constexpr int kTileTokens = 64;  // tokens per KV tile of the MFMA tile kernel (
 constexpr int kTileCols = 128;   // (q row, head) columns per tile work item (4 waves x 32)
 constexpr int kDecodeCols = 32;  // max (q row, head) columns of one decode work item (2 MFMA N blocks)
 constexpr int kDecodeWavesPerCu = 8;  // decode wavefronts resident per CU (one kv head each)
+constexpr int kShortMinWaves = 4;     // wavefronts a workgroup of the short-context kernel has at least
 
 // Per sequence, derived from the CSR metadata exactly as the reference ATen
 // plan does (portable_gpu_ops.cpp:30): len = (kv[b+1]-kv[b]-1)*page + last[b].
@@ -67,10 +68,33 @@ struct alignas(64) ShareStart {
   DecodeItem first;
   int32_t pg0;
   int32_t pg1;
-  int32_t pad[4];
+  int32_t n_short;  // in every record, so that a graph launch need not read the header first: > 0 when the
+                    // batch is planned as that many ShortItem records at the heap's start and no shares
+  int32_t pad[3];
 };
 static_assert(sizeof(ShareStart) == 64, "one 64-byte scalar load");
 static_assert(sizeof(DecodeItem) == 32, "two pieces per 64 bytes");
+
+// One workgroup's unit of the short-context kernel: query rows [q0, q0+nq)
+// (all the query heads of kv head `kvh`, at most kDecodeCols columns) against
+// tokens [t0, t1), t0 a multiple of 16; part as in WorkItem.  Its 16-token
+// blocks are divided evenly among the workgroup's W wavefronts (wavefront w:
+// blocks [w * n, (w + 1) * n) of the item, n = ceil(blocks / W)); `block`
+// names the first four of every wavefront by their index in the cache in
+// units of 16 tokens (those past a wavefront's last repeat it), so that the
+// first loads follow a single metadata read.
+struct alignas(32) ShortItem {
+  int32_t q0;
+  int32_t nq;
+  int32_t kvh;
+  int32_t vis;       // last token that row q0 sees under the causal mask
+  int32_t t0;
+  int32_t t1;
+  int32_t part;
+  int32_t page_off;  // index of the sequence's first page id
+  int32_t block[4 * kDecodeWavesPerCu];
+};
+static_assert(sizeof(ShortItem) == 160, "record and block list in two scalar loads");
 
 // One query row whose tokens were split over `nsplit` work items.  Split s
 // of this row lives in partial slot part + s*stride.
@@ -96,6 +120,8 @@ struct AttnArgs {
   const DecodeItem* ditems;  // decode only: the pieces, share by share
   const ShareStart* shares;  // decode only: one record per share
   int n_share_cap;           // decode only: records in `shares`
+  const ShortItem* shorts;   // short-context kernel: the items (graph launches: the heap's start)
+  int n_short;               // short-context kernel, eager launches: items at `shorts`
   uint16_t* part_o;        // [slots][hq][128] in the attention's 16-bit type, normalised per split
   float* part_lse;         // [slots][hq] log2 domain
   int hq;

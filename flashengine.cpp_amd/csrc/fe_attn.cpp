@@ -24,7 +24,8 @@
 #include "planner.hpp"
 
 namespace feattn {
-hipError_t launch_decode(const AttnArgs& a, bool bf16, int waves, int ncb, int causal, int grid, hipStream_t st);
+hipError_t launch_decode(const AttnArgs& a, bool bf16, int waves, int ncb, int causal, bool any, int grid,
+                         hipStream_t st);
 int decode_wg_waves(int hkv);
 hipError_t launch_tile(const AttnArgs& a, bool bf16, bool causal, bool stream, int grid, hipStream_t st);
 hipError_t launch_merge(const MergeArgs& a, bool bf16, int grid, hipStream_t st);
@@ -123,10 +124,10 @@ Layout make_layout(const Regions& r) {
 // Byte offsets of the lists inside the heap (each 256-byte aligned, so a
 // list's first record index is its offset over the record size).
 struct HeapPlace {
-  size_t pages, decode, tile[2], merge[2], used;
+  size_t shorts, pages, decode, tile[2], merge[2], used;
 };
 
-HeapPlace place_heap(size_t pages, size_t decode, const size_t tile[2], const size_t merge[2]) {
+HeapPlace place_heap(size_t shorts, size_t pages, size_t decode, const size_t tile[2], const size_t merge[2]) {
   HeapPlace p;
   size_t off = 0;
   auto put = [&](size_t bytes) {
@@ -134,6 +135,7 @@ HeapPlace place_heap(size_t pages, size_t decode, const size_t tile[2], const si
     off = align256(off + bytes);
     return at;
   };
+  p.shorts = put(sizeof(ShortItem) * shorts);  // first: a graph launch finds them without reading the header
   p.pages = put(sizeof(int32_t) * pages);
   p.decode = put(sizeof(DecodeItem) * decode);
   for (int m = 0; m < 2; ++m) p.tile[m] = put(sizeof(WorkItem) * tile[m]);
@@ -149,7 +151,7 @@ HeapPlace place_lists(const BuiltPlan& bp, int npages, const bool staged[2]) {
     tile[m] = staged[m] ? bp.mode[m].tile.size() : 0;
     merge[m] = staged[m] ? bp.mode[m].merge.size() : 0;
   }
-  return place_heap((size_t)npages, bp.decode_items.size(), tile, merge);
+  return place_heap(bp.shorts.size(), (size_t)npages, bp.decode_items.size(), tile, merge);
 }
 
 Regions capacity_regions(const PlanShape& sh) {
@@ -159,7 +161,8 @@ Regions capacity_regions(const PlanShape& sh) {
   const size_t tile[2] = {(size_t)sh.item_cap, (size_t)sh.item_cap};
   const size_t merge[2] = {(size_t)sh.partial_cap, (size_t)sh.partial_cap};
   for (int m = 0; m < 2; ++m) r.tshare[m] = (size_t)sh.tile_slots + 1;
-  r.heap = place_heap((size_t)sh.max_batch * sh.max_pages, (size_t)sh.item_cap, tile, merge).used;
+  // (short-context items take the place of decode pieces, and of less room)
+  r.heap = place_heap(0, (size_t)sh.max_batch * sh.max_pages, (size_t)sh.item_cap, tile, merge).used;
   return r;
 }
 
@@ -249,6 +252,14 @@ int write_image(uint8_t* h, const Layout& l, const HeapPlace& hp, const PlanShap
     ss[k].first = shift_piece(ss[k].first);
   }
   std::memset(ss + n_shares, 0, sizeof(ShareStart) * (size_t)(scap - n_shares));
+  const std::vector<ShortItem>& shorts = bp.shorts;
+  if (!shorts.empty())
+    for (int k = 0; k < scap; ++k) ss[k].n_short = (int32_t)shorts.size();
+  ShortItem* sp = reinterpret_cast<ShortItem*>(heap + hp.shorts);
+  for (size_t i = 0; i < shorts.size(); ++i) {
+    sp[i] = shorts[i];
+    sp[i].page_off += pages_base;
+  }
 
   const int tslots = sh.tile_slots;
   for (int m = 0; m < 2; ++m) {
@@ -290,6 +301,7 @@ struct Launch {
   int graph_stream[2] = {-1, -1};      // graph plans: that choice at the first graph prepare
   int n_decode = 0, n_tile[2] = {0, 0}, n_merge[2] = {0, 0};
   size_t merge_off[2] = {0, 0};  // heap offsets of the merge lists just staged
+  int n_short = 0;
   int n_tshare[2] = {0, 0};  // tile shares (workgroups) in use per mask mode
   int decode_wg = 8;         // wavefronts per decode workgroup
   int decode_nc = 16;
@@ -320,9 +332,17 @@ bool reads_tokens_once(const BuiltPlan& bp, const PlanShape& sh) {
   return true;
 }
 
+// Wavefronts of the short-context kernel's workgroups: those of a decode
+// workgroup, so that a graph plan's one launch serves both; 0: too few.
+int short_waves(const PlanShape& sh) {
+  const int w = decode_wg_waves(sh.hkv);
+  return w >= kShortMinWaves ? w : 0;
+}
+
 void record_lists(Launch& L, const BuiltPlan& bp, const HeapPlace& hp, int nc) {
   L.decode_nc = nc;
   for (int m = 0; m < 2; ++m) L.merge_off[m] = hp.merge[m];
+  L.n_short = (int)bp.shorts.size();
   L.n_decode = (int)bp.decode_starts.size() * L.sh.hkv;  // busy decode wavefronts
   for (int m = 0; m < 2; ++m) {
     L.n_tile[m] = (int)bp.mode[m].tile.size();
@@ -385,14 +405,18 @@ int launch_all(const Launch& L, const void* q, const void* k_cache, const void* 
   a.page_shift = shift;
   a.scale_log2 = 1.4426950408889634f / 11.313708498984761f;  // log2(e) / sqrt(128)
   hipError_t e;
-  if (L.graph || L.n_decode > 0) {
+  if (L.graph || L.n_decode > 0 || L.n_short > 0) {
     AttnArgs d = a;
     d.ditems = reinterpret_cast<const DecodeItem*>(heap);
     d.shares = reinterpret_cast<const ShareStart*>(L.dev + L.lay.shares);
     d.n_share_cap = (int)L.lay.n.shares;
     const int wv = L.decode_wg;
-    const int grid = L.graph ? L.grid_decode_cap : std::min(L.grid_decode_cap, (L.n_decode + wv - 1) / wv);
-    e = launch_decode(d, L.bf16, L.decode_wg, L.decode_nc / 16, causal ? 1 : 0, std::max(grid, 1), st);
+    d.shorts = reinterpret_cast<const ShortItem*>(heap);
+    d.n_short = L.n_short;
+    const int grid = L.graph      ? L.grid_decode_cap
+                     : d.n_short > 0 ? d.n_short
+                                     : std::min(L.grid_decode_cap, (L.n_decode + wv - 1) / wv);
+    e = launch_decode(d, L.bf16, L.decode_wg, L.decode_nc / 16, causal ? 1 : 0, L.graph, std::max(grid, 1), st);
     if (e != hipSuccess) return hip_fail(e, "decode kernel launch");
   }
   if (L.graph ? L.graph_tile > 0 : L.n_tile[mode] > 0) {
@@ -472,7 +496,7 @@ int attn_oneshot(uint8_t* arena, size_t bytes, int device, const void* q, const 
   rc = check_stream_device(st, device);
   if (rc != FE_OK) return rc;
   BuiltPlan bp;
-  rc = build_plan(sh, qo, kv, pages, last, batch, rows, bp, err);
+  rc = build_plan(sh, qo, kv, pages, last, batch, rows, bp, err, short_waves(sh));
   if (rc != FE_OK) return fail(rc, err);
   const int mode = causal ? 1 : 0;
   const int npages = batch > 0 ? kv[batch] : 0;
@@ -612,7 +636,7 @@ int fe_attn_plan_prepare(fe_attn_plan* p, const int32_t* qo, const int32_t* kv, 
   if (cap != hipStreamCaptureStatusNone)
     return fail(FE_EINVAL, "prepare_plan: the stream is capturing a graph; prepare outside the capture and "
                            "capture only the attention calls");
-  rc = build_plan(L.sh, qo, kv, pages, last, batch, rows, bp, err);
+  rc = build_plan(L.sh, qo, kv, pages, last, batch, rows, bp, err, short_waves(L.sh));
   if (rc != FE_OK) return fail(rc, err);
   int nc = bp.decode_nc;
   int graph_nc = p->graph_nc, graph_tile = L.graph_tile;

@@ -194,6 +194,102 @@ bool cut_tile_stream(const std::vector<SeqInfo>& seqs, int G, int hkv, bool caus
   return true;
 }
 
+// Plans a batch of decode sequences as short-context items, or returns false
+// (leaving `out` alone) where shares are the faster plan.
+//
+// A workgroup takes W * 64 tokens per round of loads (a "step").  Measured on
+// the MI355X, us per call over caches larger than the L2, this plan against
+// shares + merge, 8 kv heads (W = 8) and 4 query heads each unless said
+// otherwise:
+//   * sequences of one step: 9.2 / 14.8 (12 x 200), 10.3 / 15.4 (12 x 512); of
+//     two, with W = 4: 10.2 / 14.5 (12 x 512, 4 kv heads).  A second round
+//     of 8 wavefronts costs more than merging two pieces: 15.4 / 12.2 for 1
+//     x 1001 whole, cut 12.2.
+//   * cut into steps: 13.7 / 18.3 (1 x 4001), 13.8 / 17.4 (4 x 1984).
+//   * more items than resident workgroups: 17.0 / 15.9 (64 x 200) and, cut,
+//     27.9 / 22.3 (12 x 2048); only sequences of one block per wavefront
+//     still gain, 12.1 / 14.6 (64 x 64).
+//   * with more K and V per compute unit, the shares' whole-page streams win
+//     when the cache is cold: 188 KB, inside a replayed decode step, 1.6 us a
+//     layer slower so.  Two column blocks are slow on the shares (20.3 /
+//     26.9 at 182 KB, 5 rows of 5 heads), so the line is higher there.
+bool plan_short(const PlanShape& sh, const int32_t* pages, int waves, BuiltPlan& out) {
+  const int G = sh.hq / sh.hkv;
+  const int64_t slots = sh.decode_waves / waves;  // workgroups that run at once
+  const int step = 64 * waves;
+  int max_len = 0, max_cols = 0;
+  int64_t whole = 0, cut = 0, tokens = 0;  // items of either form
+  for (const SeqInfo& s : out.seqs) {
+    if (s.qlen == 0) continue;
+    if (s.qlen * G > kDecodeCols) return false;
+    max_len = std::max(max_len, s.len);
+    max_cols = std::max(max_cols, s.qlen * G);
+    whole += sh.hkv;
+    cut += (int64_t)sh.hkv * ceil_div(s.len, step);
+    tokens += s.len;
+  }
+  if (whole == 0) return false;
+  const int64_t per_cu = tokens * sh.hkv * (2 * kHeadDim * 2) / sh.num_cus;
+  const int64_t limit = max_cols <= 16 ? 144 << 10 : 256 << 10;
+  if (per_cu > limit) return false;
+  int piece;
+  if (max_len <= 512 && (whole <= slots || (max_len <= 16 * waves && whole <= 2 * slots)))
+    piece = 512;
+  else if (cut <= slots)
+    piece = step;
+  else
+    return false;
+  // Longest first: the order in which workgroups start.
+  std::vector<int> order;
+  for (int b = 0; b < (int)out.seqs.size(); ++b)
+    if (out.seqs[b].qlen > 0) order.push_back(b);
+  std::stable_sort(order.begin(), order.end(), [&](int x, int y) { return out.seqs[x].len > out.seqs[y].len; });
+  ModeLists ml;
+  std::vector<ShortItem> items;
+  items.reserve((size_t)(max_len <= piece ? whole : cut));
+  for (int b : order) {
+    const SeqInfo& s = out.seqs[b];
+    const int len = round_up(ceil_div(s.len, ceil_div(s.len, piece)), 16);  // of one piece
+    const int np = ceil_div(s.len, len);
+    int base = -1;
+    if (np > 1) {
+      base = ml.partial_rows;
+      ml.partial_rows += np * s.qlen;
+      for (int r = 0; r < s.qlen; ++r) ml.merge.push_back(MergeRow{s.qo + r, base + r, np, s.qlen});
+    }
+    for (int p = 0; p < np; ++p) {
+      ShortItem it{};
+      it.q0 = s.qo;
+      it.nq = s.qlen;
+      it.vis = s.len - s.qlen;
+      it.t0 = p * len;
+      it.t1 = std::min(s.len, it.t0 + len);
+      it.part = base < 0 ? -1 : base + p * s.qlen;
+      it.page_off = s.page_off;
+      const int nblk = ceil_div(it.t1 - it.t0, 16);
+      const int per = ceil_div(nblk, waves);
+      for (int w = 0; w * per < nblk; ++w) {
+        const int end = std::min(nblk, (w + 1) * per);
+        for (int j = 0; j < 4; ++j) {
+          const int tok = it.t0 + 16 * std::min(w * per + j, end - 1);
+          it.block[4 * w + j] = (int32_t)((uint32_t)pages[s.page_off + tok / sh.page] * (uint32_t)(sh.page / 16) +
+                                          (uint32_t)(tok % sh.page / 16));
+        }
+      }
+      for (int h = 0; h < sh.hkv; ++h) {
+        it.kvh = h;
+        items.push_back(it);
+      }
+    }
+  }
+  if (ml.partial_rows > sh.partial_cap || ml.merge.size() > (size_t)sh.partial_cap) return false;
+  out.decode_nc = max_cols <= 16 ? 16 : 32;
+  out.shorts = std::move(items);
+  out.mode[0] = ml;  // every row's tokens are one sequence's: the mask changes no list
+  out.mode[1] = std::move(ml);
+  return true;
+}
+
 }  // namespace
 
 int validate_shape(const PlanShape& sh, std::string& err) {
@@ -221,7 +317,7 @@ int validate_shape(const PlanShape& sh, std::string& err) {
 }
 
 static int build_plan_impl(const PlanShape& sh, const int32_t* qo, const int32_t* kv, const int32_t* pages,
-               const int32_t* last, int batch, int rows, BuiltPlan& out, std::string& err) {
+               const int32_t* last, int batch, int rows, BuiltPlan& out, std::string& err, int short_waves) {
   int rc = validate_shape(sh, err);
   if (rc != FE_OK) return rc;
   if (batch < 0 || rows < 0) {
@@ -283,6 +379,8 @@ static int build_plan_impl(const PlanShape& sh, const int32_t* qo, const int32_t
     err = "qo[batch] exceeds rows";
     return FE_EINVAL;
   }
+
+  if (short_waves > 0 && plan_short(sh, pages, short_waves, out)) return FE_OK;
 
   const int G = sh.hq / sh.hkv;
   const int slot_budget = sh.partial_cap;
@@ -481,9 +579,9 @@ static int build_plan_impl(const PlanShape& sh, const int32_t* qo, const int32_t
 }
 
 int build_plan(const PlanShape& sh, const int32_t* qo, const int32_t* kv, const int32_t* pages,
-               const int32_t* last, int batch, int rows, BuiltPlan& out, std::string& err) {
+               const int32_t* last, int batch, int rows, BuiltPlan& out, std::string& err, int short_waves) {
   try {
-    return build_plan_impl(sh, qo, kv, pages, last, batch, rows, out, err);
+    return build_plan_impl(sh, qo, kv, pages, last, batch, rows, out, err, short_waves);
   } catch (const std::bad_alloc&) {
     err = "out of host memory while building the work lists";
     return FE_ENOMEM;

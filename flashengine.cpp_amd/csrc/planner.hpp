@@ -41,6 +41,7 @@ struct BuiltPlan {
   std::vector<ShareStart> decode_starts;  // one per share in use
   int decode_partials = 0;
   std::vector<MergeRow> decode_merge;
+  std::vector<ShortItem> shorts;  // the whole batch as short-context items (then no other items); both masks
   int decode_nc = 16;            // 16 or 32 columns per decode item (MFMA column blocks x 16)
   ModeLists mode[2];             // [0] full (non-causal), [1] causal
 };
@@ -58,7 +59,11 @@ void assign_shares(std::vector<WorkItem>& items, int slots, std::vector<int32_t>
 
 // Returns 0 (FE_OK) or a negative FE_E* code with `err` set.
 int validate_shape(const PlanShape& sh, std::string& err);
+//
+// short_waves > 0: a batch of decode sequences that is faster so is planned
+// as short-context items for workgroups of that many wavefronts
+// (`shorts`) instead of decode shares.
 int build_plan(const PlanShape& sh, const int32_t* qo, const int32_t* kv, const int32_t* pages,
-               const int32_t* last, int batch, int rows, BuiltPlan& out, std::string& err);
+               const int32_t* last, int batch, int rows, BuiltPlan& out, std::string& err, int short_waves = 0);
 
 }  // namespace feattn

@@ -1,0 +1,94 @@
+"""Short-context plans (planner.cpp: plan_short): the item lists over random
+batches, built with AddressSanitizer and UndefinedBehaviorSanitizer
+(tests/cpp/short_check.cpp), and on the GPU the kernel's edges against the
+oracle."""
+import os
+import shutil
+import subprocess
+
+import pytest
+import torch
+
+import feattn
+from feattn import workloads as W
+from oracle import aten_attention as A
+
+ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
+
+
+@pytest.mark.skipif(shutil.which("g++") is None, reason="no host C++ compiler")
+def test_short_items_cover_the_batch(tmp_path):
+    exe = tmp_path / "short_check"
+    subprocess.run(["g++", "-std=c++17", "-O1", "-g", "-fsanitize=address,undefined", "-fno-sanitize-recover=all",
+                    "-I" + os.path.join(ROOT, "include"), "-I" + os.path.join(ROOT, "flashengine.cpp_amd", "csrc"),
+                    os.path.join(ROOT, "tests", "cpp", "short_check.cpp"),
+                    os.path.join(ROOT, "flashengine.cpp_amd", "csrc", "planner.cpp"), "-o", str(exe)],
+                   check=True, timeout=300)
+    r = subprocess.run([str(exe)], capture_output=True, text=True, timeout=300)
+    assert r.returncode == 0, r.stdout + r.stderr
+
+
+# Context lengths around one block, one block per wavefront, one round of
+# loads (64 tokens per wavefront) and the longest uncut sequence of 8- and
+# 4-wavefront workgroups (hkv 8 and 4), and cut ones.
+LENS = {8: [1, 15, 16, 17, 127, 128, 129, 511, 512, 513, 640, 1023, 1024, 1025, 2100],
+        4: [1, 16, 33, 63, 64, 65, 255, 256, 257, 500, 512, 513, 1300]}
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("hq,hkv,rows,page", [(32, 8, 1, 16), (16, 8, 1, 64), (40, 8, 5, 16), (8, 8, 8, 32),
+                                              (32, 8, 8, 16), (32, 4, 1, 16), (32, 4, 4, 32), (64, 4, 1, 16)])
+@pytest.mark.parametrize("dtype,causal", [("bf16", True), ("f16", False)])
+def test_short_kernel_edges(dev, hq, hkv, rows, page, dtype, causal):
+    """All the lengths in one batch (cut into pieces and merged), then the
+    uncut ones; eagerly and replayed from a graph captured on another batch.
+    Everything a call may not read -- cache rows past a sequence's end and
+    pages of no sequence -- is NaN.  The tolerance is the one of the other
+    attention tests: 16-bit probabilities and outputs."""
+    step = 64 * hkv
+    plan = feattn.Plan(hq, hkv, 128, page, 16, 2200 // page + 2, dtype == "bf16", 12000 // page)
+    graph_plan = feattn.Plan(hq, hkv, 128, page, 16, 2200 // page + 2, dtype == "bf16", 12000 // page)
+    graph = None
+    for lens in (LENS[hkv], [n for n in LENS[hkv] if n <= 2 * step], [2 * step]):
+        lens = [max(n, rows) for n in lens]
+        b = W.make_batch(hq, hkv, starts=[n - rows for n in lens], qlens=[rows] * len(lens), seed=len(lens),
+                         page=page, pool=12000 // page)
+        q, kc, vc = W.make_tensors(b, seed=7, dtype=dtype)
+        want, want_lse = A.run(b, q, kc, vc, causal)
+        used = torch.zeros((b.blocks + 1) * page, dtype=torch.bool)
+        for s in range(b.batch):
+            for t in range(b.lens[s]):
+                used[b.tables[s][t // page] * page + t % page] = True
+        used = used.view(b.blocks + 1, page)
+        kc[~used] = float("nan")
+        vc[~used] = float("nan")
+        kd, vd, qd = kc.to(dev), vc.to(dev), q.to(dev)
+
+        def run(p):
+            out = torch.full_like(qd, float("nan"))
+            lse = torch.full((b.rows, hq), float("nan"), device=dev)
+            p.run(qd, kd, vd, out, causal=causal, lse=lse)
+            return out, lse
+
+        plan.prepare(b.qo, b.kv, b.pages, b.last, b.batch, b.rows)
+        graph_plan.prepare(b.qo, b.kv, b.pages, b.last, b.batch, b.rows, graph=True)
+        got = [run(plan), run(graph_plan)]
+        if graph is None:
+            sq, sk, sv = qd.clone(), kd.clone(), vd.clone()
+            so, sl = torch.full_like(sq, float("nan")), torch.full((b.rows, hq), float("nan"), device=dev)
+            torch.cuda.synchronize()
+            graph = torch.cuda.CUDAGraph()
+            with torch.cuda.graph(graph):
+                graph_plan.run(sq, sk, sv, so, causal=causal, lse=sl)
+        sq[:b.rows].copy_(qd)
+        sk.copy_(kd)
+        sv.copy_(vd)
+        graph.replay()
+        got.append((so[:b.rows].clone(), sl[:b.rows].clone()))
+        torch.cuda.synchronize()
+        for out, lse in got:
+            torch.testing.assert_close(out.float().cpu(), want.float(), atol=1e-2, rtol=1e-2)
+            torch.testing.assert_close(lse.cpu(), want_lse, atol=1e-3, rtol=0)
+            assert torch.equal(out, got[0][0]) and torch.equal(lse, got[0][1])
+    plan.close()
+    graph_plan.close()
