@@ -727,72 +727,137 @@ __global__ __launch_bounds__(256, 2) void attn_tile_kernel(AttnArgs a) {
 // ===========================================================================
 // Split-KV merge
 // ===========================================================================
-// One wavefront per (merged row, pair of heads): lanes 0-31 take head 2hp,
-// lanes 32-63 head 2hp + 1, each lane 4 of the 128 dims, so every partial-row
-// load is one 8-byte access per lane.  Splits are folded in batches of
-// kMergeBatch whose log-sum-exps and partial rows are all in flight
-// together; loads past a row's split count are not issued.
+// Per (merged row, pair of heads): lanes 0-31 take head 2hp, lanes 32-63 head
+// 2hp + 1, each lane 4 of the 128 dims, so every partial-row load is one
+// 8-byte access per lane.  Splits are folded in batches whose log-sum-exps and
+// partial rows are all in flight together.  What bounds it is that chain of round trips, not bytes:
+//   * narrow: one wavefront per pair, one batch of 4 or batches of 8, for the many rows of few
+//     splits that a full decode batch or prefill leaves.
+//   * wide: the four wavefronts of a workgroup fold a pair's splits together,
+//     batches of 16 each, and are combined in LDS.  One sequence of 16001
+//     tokens is 128 splits, 16 round trips in the narrow form.
+struct MergeState {
+  float m, wsum;  // log2-domain maximum, sum of weights relative to it
+  f32x4 acc;
+};
+
+__device__ __forceinline__ MergeRow ldc_merge(const MergeRow* rows, int i) {
+  const int32_t* p = reinterpret_cast<const int32_t*>(rows + uniform(i));
+  return MergeRow{ldc(p, 0), ldc(p, 1), ldc(p, 2), ldc(p, 3)};
+}
+
+template <bool BF16, int BATCH>
+__device__ __forceinline__ void merge_fold(const MergeArgs& a, const MergeRow& mr, int head, int d, int sp0,
+                                           MergeState& s) {
+  float l[BATCH];
+  u32x2 rv[BATCH];  // four 16-bit partial values
+  // Past the last split the loads repeat it (a cache hit) and its weight is
+  // zero: a branch around each load lets the compiler move the 16-bit
+  // conversions into it, behind a wait per load (verify rows in fp16: the
+  // call took 66.9 us so, 63.6 without).
+#pragma unroll
+  for (int u = 0; u < BATCH; ++u) {
+    const size_t slot = (size_t)(mr.part + min(sp0 + u, mr.nsplit - 1) * mr.stride);
+    l[u] = a.part_lse[slot * a.hq + head];
+    rv[u] = *reinterpret_cast<const u32x2*>(a.part_o + (slot * a.hq + head) * kHeadDim + d);
+  }
+#pragma unroll
+  for (int u = 0; u < BATCH; ++u)
+    if (sp0 + u >= mr.nsplit) l[u] = kNegInf;
+  float bm = s.m;
+#pragma unroll
+  for (int u = 0; u < BATCH; ++u) bm = fmaxf(bm, l[u]);
+  const float mu = bm == kNegInf ? 0.f : bm;
+  const float sc = fast_exp2(s.m - mu);
+  s.wsum *= sc;
+  s.acc *= sc;
+#pragma unroll
+  for (int u = 0; u < BATCH; ++u) {
+    const float wt = fast_exp2(l[u] - mu);
+    const f32x4 v = {lo_f32<BF16>(rv[u][0]), hi_f32<BF16>(rv[u][0]), lo_f32<BF16>(rv[u][1]),
+                     hi_f32<BF16>(rv[u][1])};
+    s.wsum += wt;
+    s.acc += wt * v;
+  }
+  s.m = bm;
+}
+
 template <bool BF16>
+__device__ __forceinline__ void merge_write(const MergeArgs& a, int row, int head, int d, const MergeState& s) {
+  const float inv = s.wsum > 0.f ? 1.f / s.wsum : 0.f;
+  const size_t oi = (size_t)row * a.hq + head;
+  const u32x2 o = {pack2<BF16>(s.acc[0] * inv, s.acc[1] * inv), pack2<BF16>(s.acc[2] * inv, s.acc[3] * inv)};
+  *reinterpret_cast<u32x2*>(a.out + oi * kHeadDim + d) = o;
+  if (a.lse != nullptr && d == 0) a.lse[oi] = s.wsum > 0.f ? (s.m + __log2f(s.wsum)) * kLn2 : kNegInf;
+}
+
+// A graph launch (Header) folds the list of the latest prepare in the form the
+// header names; an eager launch is handed the list and its length.
+enum class MergeForm { Narrow, Wide, Header };
+
+template <bool BF16, MergeForm FORM>
 __global__ __launch_bounds__(256) void attn_merge_kernel(MergeArgs a) {
+  constexpr int WAVES = 4, kFew = 4, kNarrow = 8, kWide = 16;
   const int lane = threadIdx.x & 63;
-  const int hq = a.hq;
-  const int hpairs = (hq + 1) >> 1;
-  const int stride = gridDim.x * 4;
-  // A graph launch folds the list of the latest prepare, found through the
-  // header; an eager launch is handed the list and its length.
+  const int wave = uniform(threadIdx.x >> 6);
+  const int hpairs = (a.hq + 1) >> 1;
   const MergeRow* rows = a.rows;
   int n_rows = a.n_rows;
-  if (a.count_base != nullptr) {
+  bool wide = FORM == MergeForm::Wide;
+  if constexpr (FORM == MergeForm::Header) {
     n_rows = uniform(a.count_base[0]);
     rows += uniform(a.count_base[1]);
+    wide = uniform(a.count_base[2]) != 0;
   }
   const int n_pairs = n_rows * hpairs;
   const int d = 4 * (lane & 31);
-  for (int pair = blockIdx.x * 4 + uniform(threadIdx.x >> 6); pair < n_pairs; pair += stride) {
-    const MergeRow mr = rows[pair / hpairs];
+  if (FORM != MergeForm::Wide && !wide) {
+    for (int pair = blockIdx.x * WAVES + wave; pair < n_pairs; pair += gridDim.x * WAVES) {
+      const MergeRow mr = ldc_merge(rows, pair / hpairs);
+      const int h = 2 * (pair % hpairs) + (lane >> 5);
+      const int hh = h < a.hq ? h : a.hq - 1;
+      MergeState s{kNegInf, 0.f, {0.f, 0.f, 0.f, 0.f}};
+      if (mr.nsplit <= kFew) {
+        merge_fold<BF16, kFew>(a, mr, hh, d, 0, s);
+      } else {
+        for (int sp0 = 0; sp0 < mr.nsplit; sp0 += kNarrow) merge_fold<BF16, kNarrow>(a, mr, hh, d, sp0, s);
+      }
+      if (h < a.hq) merge_write<BF16>(a, mr.row, h, d, s);
+    }
+    return;
+  }
+  if constexpr (FORM == MergeForm::Narrow) return;
+  __shared__ f32x4 sh_acc[WAVES][64];
+  __shared__ float sh_m[WAVES][2], sh_w[WAVES][2];
+  for (int pair = blockIdx.x; pair < n_pairs; pair += gridDim.x) {
+    const MergeRow mr = ldc_merge(rows, pair / hpairs);
     const int h = 2 * (pair % hpairs) + (lane >> 5);
-    const bool on = h < hq;
-    const int hh = on ? h : hq - 1;
-    constexpr int kMergeBatch = 8;
-    float m = kNegInf, wsum = 0.f;
-    f32x4 acc = {0.f, 0.f, 0.f, 0.f};
-    for (int sp0 = 0; sp0 < mr.nsplit; sp0 += kMergeBatch) {
-      float l[kMergeBatch];
-      u32x2 rv[kMergeBatch];  // four 16-bit partial values
-#pragma unroll
-      for (int u = 0; u < kMergeBatch; ++u) {
-        l[u] = kNegInf;
-        rv[u] = u32x2{0u, 0u};
-        if (sp0 + u < mr.nsplit) {  // wave-uniform
-          const size_t slot = (size_t)(mr.part + (sp0 + u) * mr.stride);
-          l[u] = a.part_lse[slot * hq + hh];
-          rv[u] = *reinterpret_cast<const u32x2*>(a.part_o + (slot * hq + hh) * kHeadDim + d);
-        }
-      }
-      float bm = m;
-#pragma unroll
-      for (int u = 0; u < kMergeBatch; ++u) bm = fmaxf(bm, l[u]);
-      const float mu = bm == kNegInf ? 0.f : bm;
-      const float sc = fast_exp2(m - mu);
-      wsum *= sc;
-      acc *= sc;
-#pragma unroll
-      for (int u = 0; u < kMergeBatch; ++u) {
-        const float wt = fast_exp2(l[u] - mu);
-        const f32x4 v = {lo_f32<BF16>(rv[u][0]), hi_f32<BF16>(rv[u][0]), lo_f32<BF16>(rv[u][1]),
-                         hi_f32<BF16>(rv[u][1])};
-        wsum += wt;
-        acc += wt * v;
-      }
-      m = bm;
+    MergeState s{kNegInf, 0.f, {0.f, 0.f, 0.f, 0.f}};
+    for (int sp0 = kWide * wave; sp0 < mr.nsplit; sp0 += kWide * WAVES)
+      merge_fold<BF16, kWide>(a, mr, h < a.hq ? h : a.hq - 1, d, sp0, s);
+    sh_acc[wave][lane] = s.acc;
+    if (d == 0) {
+      sh_m[wave][lane >> 5] = s.m;
+      sh_w[wave][lane >> 5] = s.wsum;
     }
-    if (on) {
-      const float inv = wsum > 0.f ? 1.f / wsum : 0.f;
-      const size_t oi = (size_t)mr.row * hq + h;
-      const u32x2 o = {pack2<BF16>(acc[0] * inv, acc[1] * inv), pack2<BF16>(acc[2] * inv, acc[3] * inv)};
-      *reinterpret_cast<u32x2*>(a.out + oi * kHeadDim + d) = o;
-      if (a.lse != nullptr && (lane & 31) == 0) a.lse[oi] = wsum > 0.f ? (m + __log2f(wsum)) * kLn2 : kNegInf;
+    __syncthreads();
+    if (wave == 0) {
+      float m[WAVES], top = kNegInf;
+#pragma unroll
+      for (int w = 0; w < WAVES; ++w) {
+        m[w] = sh_m[w][lane >> 5];
+        top = fmaxf(top, m[w]);
+      }
+      MergeState t{top, 0.f, {0.f, 0.f, 0.f, 0.f}};
+#pragma unroll
+      for (int w = 0; w < WAVES; ++w) {
+        const float wt = fast_exp2(m[w] - (top == kNegInf ? 0.f : top));
+        t.wsum += wt * sh_w[w][lane >> 5];
+        t.acc += wt * sh_acc[w][lane];
+      }
+      if (h < a.hq) merge_write<BF16>(a, mr.row, h, d, t);
     }
+    __syncthreads();
   }
 }
 
@@ -890,9 +955,19 @@ hipError_t launch_stage_copy(void* dst, const void* src, size_t bytes, hipStream
   return hipGetLastError();
 }
 
+template <bool BF16>
+static void merge_launch(const MergeArgs& a, int grid, hipStream_t st) {
+  if (a.count_base != nullptr)
+    hipLaunchKernelGGL((attn_merge_kernel<BF16, MergeForm::Header>), dim3(grid), dim3(256), 0, st, a);
+  else if (a.wide)
+    hipLaunchKernelGGL((attn_merge_kernel<BF16, MergeForm::Wide>), dim3(grid), dim3(256), 0, st, a);
+  else
+    hipLaunchKernelGGL((attn_merge_kernel<BF16, MergeForm::Narrow>), dim3(grid), dim3(256), 0, st, a);
+}
+
 hipError_t launch_merge(const MergeArgs& a, bool bf16, int grid, hipStream_t st) {
-  if (bf16) hipLaunchKernelGGL((attn_merge_kernel<true>), dim3(grid), dim3(256), 0, st, a);
-  else hipLaunchKernelGGL((attn_merge_kernel<false>), dim3(grid), dim3(256), 0, st, a);
+  if (bf16) merge_launch<true>(a, grid, st);
+  else merge_launch<false>(a, grid, st);
   return hipGetLastError();
 }
 

@@ -136,7 +136,8 @@ struct MergeArgs {
   float* lse;
   const MergeRow* rows;       // the records (eager launches) or the list they are indexed from (graph launches)
   int n_rows;                 // eager launches: records at `rows`
-  const int32_t* count_base;  // graph launches, device-resident: records to fold, index of the first in `rows`
+  int wide;                   // eager launches: a workgroup per (row, head pair) instead of a wavefront
+  const int32_t* count_base;  // graph launches, device-resident: records to fold, index of the first in `rows`, wide
   const uint16_t* part_o;
   const float* part_lse;
   int hq;

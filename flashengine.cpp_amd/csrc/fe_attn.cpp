@@ -167,14 +167,29 @@ Regions capacity_regions(const PlanShape& sh) {
 }
 
 // header[] indices.  Tile ends are heap indices (a workgroup's items end at
-// min(tile_off[b + 1], end)); each merge count is followed by its base.
+// min(tile_off[b + 1], end)); each merge count is followed by its base and
+// the form of the merge kernel.
 enum {
   kHdrDecodeShares = 0,
   kHdrTileEnd0 = 2,
   kHdrTileEnd1 = 3,
-  kHdrMerge0 = 4,  // count, base
-  kHdrMerge1 = 6,  // count, base
+  kHdrMerge0 = 4,  // count, base, wide
+  kHdrMerge1 = 8,  // count, base, wide
 };
+
+// Whether a merge list is folded by a workgroup per (row, pair of heads)
+// (attn_merge_kernel): for rows of more splits than a wavefront has in flight
+// at once, while four such workgroups per compute unit hold them all.  Against
+// a wavefront each: one sequence of 16001 tokens, 32/8 heads, 41.4 -> 21.1 us a
+// call (16 pairs of 128 splits); 8 sequences of ~3000, 5 rows of 40/8 heads,
+// 33.1 -> 31.7 (800 pairs of ~7-15 splits); with no row above 8 splits both
+// make one round trip and the wavefront form needs a quarter of the workgroups.
+bool merge_wide(const std::vector<MergeRow>& rows, const PlanShape& sh) {
+  if ((int64_t)rows.size() * ((sh.hq + 1) / 2) > (int64_t)sh.num_cus * 4) return false;
+  for (const MergeRow& r : rows)
+    if (r.nsplit > 8) return true;
+  return false;
+}
 
 // Validated shape (host-only sizes).
 int make_shape(int hq, int hkv, int dim, int page, int max_batch, int max_pages, int blocks, PlanShape& sh,
@@ -270,6 +285,7 @@ int write_image(uint8_t* h, const Layout& l, const HeapPlace& hp, const PlanShap
     hdr[m ? kHdrTileEnd1 : kHdrTileEnd0] = tile_base + n_tile;
     hdr[(m ? kHdrMerge1 : kHdrMerge0) + 0] = (int32_t)n_merge;
     hdr[(m ? kHdrMerge1 : kHdrMerge0) + 1] = (int32_t)(hp.merge[m] / sizeof(MergeRow));
+    hdr[(m ? kHdrMerge1 : kHdrMerge0) + 2] = merge_wide(bp.mode[m].merge, sh) ? 1 : 0;
     if (n_tile > 0) std::memcpy(heap + hp.tile[m], bp.mode[m].tile.data(), sizeof(WorkItem) * n_tile);
     if (n_merge > 0) std::memcpy(heap + hp.merge[m], bp.mode[m].merge.data(), sizeof(MergeRow) * n_merge);
     // share offsets up to the launch capacity: shares past those in use are
@@ -300,6 +316,8 @@ struct Launch {
   bool tile_stream[2] = {true, true};  // tile K/V reads with the non-temporal hint, per mask mode
   int graph_stream[2] = {-1, -1};      // graph plans: that choice at the first graph prepare
   int n_decode = 0, n_tile[2] = {0, 0}, n_merge[2] = {0, 0};
+  bool wide_merge[2] = {false, false};
+  int64_t rows = 0;  // query rows of the sequences
   size_t merge_off[2] = {0, 0};  // heap offsets of the merge lists just staged
   int n_short = 0;
   int n_tshare[2] = {0, 0};  // tile shares (workgroups) in use per mask mode
@@ -340,6 +358,8 @@ int short_waves(const PlanShape& sh) {
 }
 
 void record_lists(Launch& L, const BuiltPlan& bp, const HeapPlace& hp, int nc) {
+  L.rows = 0;
+  for (const SeqInfo& s : bp.seqs) L.rows += s.qlen;
   L.decode_nc = nc;
   for (int m = 0; m < 2; ++m) L.merge_off[m] = hp.merge[m];
   L.n_short = (int)bp.shorts.size();
@@ -348,6 +368,7 @@ void record_lists(Launch& L, const BuiltPlan& bp, const HeapPlace& hp, int nc) {
     L.n_tile[m] = (int)bp.mode[m].tile.size();
     L.n_tshare[m] = bp.mode[m].tile_off.empty() ? 0 : (int)bp.mode[m].tile_off.size() - 1;
     L.n_merge[m] = (int)bp.mode[m].merge.size();
+    L.wide_merge[m] = merge_wide(bp.mode[m].merge, L.sh);
     // Graph plans keep the policy their tile launch was captured with (a
     // cache hint: results do not depend on it).
     const bool once = reads_tokens_once(bp, L.sh);
@@ -442,8 +463,17 @@ int launch_all(const Launch& L, const void* q, const void* k_cache, const void* 
     m.part_o = L.part_o;
     m.part_lse = L.part_lse;
     m.hq = L.sh.hq;
-    const int pairs4 = (int)(((int64_t)L.n_merge[mode] * ((L.sh.hq + 1) / 2) + 3) / 4);
-    const int grid = L.graph ? L.grid_merge_cap : std::min(L.grid_merge_cap, pairs4);
+    // Row and head-pair units, one per workgroup (wide) or per wavefront.  A
+    // graph launch gets a workgroup per unit that the query rows of the
+    // latest prepare can need, and loops where a later one needs more (2048
+    // workgroups, mostly idle, took 2 us longer in a decode step of 12
+    // sequences).
+    const int64_t hpairs = (L.sh.hq + 1) / 2;
+    m.wide = L.wide_merge[mode] ? 1 : 0;
+    const int64_t wgs = L.graph    ? L.rows * hpairs
+                        : m.wide ? L.n_merge[mode] * hpairs
+                                 : (L.n_merge[mode] * hpairs + 3) / 4;
+    const int grid = (int)std::min<int64_t>(L.grid_merge_cap, wgs);
     e = launch_merge(m, L.bf16, std::max(grid, 1), st);
     if (e != hipSuccess) return hip_fail(e, "merge kernel launch");
   }

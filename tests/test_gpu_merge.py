@@ -1,0 +1,44 @@
+"""Split-KV merge at the edges of its batches: splits per row around 8 (one
+batch of a wavefront), 16 and 64 (one batch of each wavefront of a workgroup)
+and an odd head count, eagerly and from a graph plan whose launch serves both
+forms, against the oracle (tolerance of the attention tests: 16-bit partial
+rows and outputs)."""
+import pytest
+import torch
+
+import feattn
+from feattn import workloads as W
+from oracle import aten_attention as A
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("dtype", ["bf16", "f16"])
+@pytest.mark.parametrize("rows", [1, 3])
+def test_split_counts(dev, dtype, rows):
+    # 5 kv heads: workgroups of one wavefront and shares of 64 tokens, so a
+    # sequence alone is cut into ceil(tokens / 64) splits.
+    hq = hkv = 5
+    plan = feattn.Plan(hq, hkv, 128, 16, 2, 600, dtype == "bf16", 1200)
+    graph_plan = feattn.Plan(hq, hkv, 128, 16, 2, 600, dtype == "bf16", 1200)
+    for lens in ([64 * 130 + 7], [64 * 8], [64 * 8 + 1], [64 * 16 + 1], [64 * 64], [64 * 64 + 1], [70, 64 * 17]):
+        b = W.make_batch(hq, hkv, starts=[n - rows for n in lens], qlens=[rows] * len(lens), seed=lens[0], pool=1200)
+        counts = feattn.describe(hq, hkv, 128, 16, 2, 600, 1200, b.qo, b.kv, b.pages, b.last, b.batch, b.rows)
+        if len(lens) == 1:
+            assert counts[3] == -(-lens[0] // 64) * rows  # partial rows
+        q, kc, vc = W.make_tensors(b, seed=3, dtype=dtype)
+        want, want_lse = A.run(b, q, kc, vc, True)
+        q, kc, vc = q.to(dev), kc.to(dev), vc.to(dev)
+        got = []
+        for p, graph in ((plan, False), (graph_plan, True)):
+            p.prepare(b.qo, b.kv, b.pages, b.last, b.batch, b.rows, graph=graph)
+            out = torch.full_like(q, float("nan"))
+            lse = torch.full((b.rows, hq), float("nan"), device=dev)
+            p.run(q, kc, vc, out, causal=True, lse=lse)
+            torch.cuda.synchronize()
+            torch.testing.assert_close(out.float().cpu(), want.float(), atol=1e-2, rtol=1e-2)
+            torch.testing.assert_close(lse.cpu(), want_lse, atol=1e-3, rtol=0)
+            got.append((out, lse))
+        assert torch.equal(got[0][0], got[1][0]) and torch.equal(got[0][1], got[1][1])
+    plan.close()
+    graph_plan.close()
