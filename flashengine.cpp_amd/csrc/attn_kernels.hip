@@ -139,12 +139,12 @@ __global__ __launch_bounds__(64 * WAVES, ANY ? 2 : 1) void attn_decode_kernel(At
   // Per-lane pieces of the copy and read addresses (fixed for the kernel).
   // Copy instruction r, lane i = 16*J + L: row 4r + J, chunk position L.
   const int row_bytes = a.hkv * kHeadDim * 2;
-  int k_goff[4], v_goff[4];
+  uint32_t k_goff[4], v_goff[4];
 #pragma unroll
   for (int r = 0; r < 4; ++r) {
     const int t = 4 * r + J;
-    k_goff[r] = t * row_bytes + 16 * (L ^ t);
-    v_goff[r] = t * row_bytes + 16 * (L ^ ((2 * t) & 15));
+    k_goff[r] = (uint32_t)(t * row_bytes + 16 * (L ^ t));
+    v_goff[r] = (uint32_t)(t * row_bytes + 16 * (L ^ ((2 * t) & 15)));
   }
   // K operand for k-step s: token L, chunk 4s + J; Q operand: column L, same chunk.
   uint32_t k_lds[4];
@@ -210,7 +210,7 @@ __global__ __launch_bounds__(64 * WAVES, ANY ? 2 : 1) void attn_decode_kernel(At
       pg_cur = pg_next;
       const char* kb = block_addr(a.kc, c_tok, pg_cur);
 #pragma unroll
-      for (int r = 0; r < 4; ++r) lds_dma16<true>(kb + k_goff[r], dst + 1024 * r);
+      for (int r = 0; r < 4; ++r) lds_dma16<true>(kb, k_goff[r], dst + 1024 * r);
       // page of the next K block: later in this item, or the next item's first
       if (first_k) {
         pg_next = pg_after;
@@ -224,7 +224,7 @@ __global__ __launch_bounds__(64 * WAVES, ANY ? 2 : 1) void attn_decode_kernel(At
     } else {
       const char* vb = block_addr(a.vc, c_tok, pg_cur);
 #pragma unroll
-      for (int r = 0; r < 4; ++r) lds_dma16<true>(vb + v_goff[r], dst + 1024 * r);
+      for (int r = 0; r < 4; ++r) lds_dma16<true>(vb, v_goff[r], dst + 1024 * r);
       c_tok += 16;
       c_kind = 1;
       if (c_tok >= cw.t1) {
@@ -433,7 +433,7 @@ constexpr int kTileBlock = 4096;               // 16 tokens x 256 bytes
 constexpr int kTileStage = 8 * kTileBlock;     // K blocks 0..3, then V blocks 0..3
 
 struct TileLanes {
-  int k_goff[4], v_goff[4];
+  uint32_t k_goff[4], v_goff[4];
   uint32_t k_lds[4], v_lds[8];
 };
 
@@ -454,9 +454,9 @@ __device__ __forceinline__ void tile_copy(const AttnArgs& a, const WorkItem& w, 
   const char* vb = reinterpret_cast<const char*>(a.vc) + blk;
   const uint32_t st = lbase + (uint32_t)(stage * kTileStage);
 #pragma unroll
-  for (int r = 0; r < 4; ++r) lds_dma16<STREAM>(kb + tl.k_goff[r], st + wave * kTileBlock + 1024 * r);
+  for (int r = 0; r < 4; ++r) lds_dma16<STREAM>(kb, tl.k_goff[r], st + wave * kTileBlock + 1024 * r);
 #pragma unroll
-  for (int r = 0; r < 4; ++r) lds_dma16<STREAM>(vb + tl.v_goff[r], st + (4 + wave) * kTileBlock + 1024 * r);
+  for (int r = 0; r < 4; ++r) lds_dma16<STREAM>(vb, tl.v_goff[r], st + (4 + wave) * kTileBlock + 1024 * r);
 }
 
 // Computes item w whose first tile was already requested into stage
@@ -680,8 +680,8 @@ __global__ __launch_bounds__(256, 2) void attn_tile_kernel(AttnArgs a) {
 #pragma unroll
   for (int r = 0; r < 4; ++r) {
     const int t = 4 * r + J;
-    tl.k_goff[r] = t * row_bytes + 16 * (L ^ t);
-    tl.v_goff[r] = t * row_bytes + 16 * (L ^ ((2 * t) & 15));
+    tl.k_goff[r] = (uint32_t)(t * row_bytes + 16 * (L ^ t));
+    tl.v_goff[r] = (uint32_t)(t * row_bytes + 16 * (L ^ ((2 * t) & 15)));
   }
 #pragma unroll
   for (int s = 0; s < 4; ++s) tl.k_lds[s] = (uint32_t)(16 * (16 * L + (((4 * s + J) ^ L) & 15)));

@@ -106,7 +106,7 @@ __device__ __forceinline__ void short_items(const AttnArgs& a, int causal, int n
           if (i < live) {
 #pragma unroll
             for (int r = 0; r < 4; ++r)
-              lds_dma16(vhead + blk[i] + v_goff[r], vst + (uint32_t)(i * kShortBlock + 1024 * r));
+              lds_dma16(vhead + blk[i], v_goff[r], vst + (uint32_t)(i * kShortBlock + 1024 * r));
           }
       };
 #pragma unroll

@@ -52,6 +52,7 @@ __device__ __forceinline__ void lds_dma16(const void* gaddr, uint32_t lds_addr) 
     asm volatile(
         "s_mov_b32 %0, m0\n\t"
         "s_mov_b32 m0, %2\n\t"
+        "s_nop 0\n\t"
         "global_load_lds_dwordx4 %1, off nt\n\t"
         "s_mov_b32 m0, %0"
         : "=&s"(saved)
@@ -61,10 +62,37 @@ __device__ __forceinline__ void lds_dma16(const void* gaddr, uint32_t lds_addr) 
     asm volatile(
         "s_mov_b32 %0, m0\n\t"
         "s_mov_b32 m0, %2\n\t"
+        "s_nop 0\n\t"
         "global_load_lds_dwordx4 %1, off\n\t"
         "s_mov_b32 m0, %0"
         : "=&s"(saved)
         : "v"(gaddr), "s"(__builtin_amdgcn_readfirstlane(lds_addr))  // wave-uniform by construction
+        : "memory");
+  }
+}
+
+// The same from a wave-uniform base and a 32-bit byte offset per lane: no
+// 64-bit address per lane to compute.  m0 is not saved: gfx9's LDS
+// instructions do not read it, and the compiler holds no value there (it
+// writes m0 right before an instruction of its own that reads it).
+template <bool STREAM = false>
+__device__ __forceinline__ void lds_dma16(const char* base, uint32_t off, uint32_t lds_addr) {
+  const uint32_t m = __builtin_amdgcn_readfirstlane(lds_addr);
+  if constexpr (STREAM) {
+    asm volatile(
+        "s_mov_b32 m0, %1\n\t"
+        "s_nop 0\n\t"
+        "global_load_lds_dwordx4 %0, %2 nt"
+        :
+        : "v"(off), "s"(m), "s"(base)
+        : "memory");
+  } else {
+    asm volatile(
+        "s_mov_b32 m0, %1\n\t"
+        "s_nop 0\n\t"
+        "global_load_lds_dwordx4 %0, %2"
+        :
+        : "v"(off), "s"(m), "s"(base)
         : "memory");
   }
 }
