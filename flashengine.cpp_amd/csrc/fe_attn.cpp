@@ -338,15 +338,13 @@ void init_launch(Launch& L, const PlanShape& sh, bool bf16) {
 // Launch sizes of the lists just staged.
 // Whether the tile lists read each K/V token once per kv head: no sequence
 // with tile work is cut into several column blocks (the planner gives such a
-// sequence ceil(qlen / (kTileCols / group)) blocks, every one over the same
-// tokens).  Chunked prefill is cut so, and those re-reads are L2 hits with
+// sequence ceil(qlen / tile_rows) blocks, every one over the same tokens).  Chunked prefill is cut so, and those re-reads are L2 hits with
 // the default policy (the 8192-token prefill takes 0.257 ms so, 0.282 ms
 // streamed); DFlash blocks and short verify rows are one block each.
-bool reads_tokens_once(const BuiltPlan& bp, const PlanShape& sh) {
+bool reads_tokens_once(const BuiltPlan& bp, const PlanShape& sh, int mode) {
   const int group = sh.hq / sh.hkv;
-  const int rows_per_block = kTileCols / group;
   for (const SeqInfo& s : bp.seqs)
-    if (s.qlen * group > kDecodeCols && s.qlen > rows_per_block) return false;
+    if (s.qlen * group > kDecodeCols && s.qlen > bp.mode[mode].tile_rows) return false;
   return true;
 }
 
@@ -371,7 +369,7 @@ void record_lists(Launch& L, const BuiltPlan& bp, const HeapPlace& hp, int nc) {
     L.wide_merge[m] = merge_wide(bp.mode[m].merge, L.sh);
     // Graph plans keep the policy their tile launch was captured with (a
     // cache hint: results do not depend on it).
-    const bool once = reads_tokens_once(bp, L.sh);
+    const bool once = reads_tokens_once(bp, L.sh, m);
     if (L.graph && L.graph_stream[m] < 0) L.graph_stream[m] = once ? 1 : 0;
     L.tile_stream[m] = L.graph ? L.graph_stream[m] > 0 : once;
   }
@@ -526,7 +524,7 @@ int attn_oneshot(uint8_t* arena, size_t bytes, int device, const void* q, const 
   rc = check_stream_device(st, device);
   if (rc != FE_OK) return rc;
   BuiltPlan bp;
-  rc = build_plan(sh, qo, kv, pages, last, batch, rows, bp, err, short_waves(sh));
+  rc = build_plan(sh, qo, kv, pages, last, batch, rows, bp, err, short_waves(sh), true);
   if (rc != FE_OK) return fail(rc, err);
   const int mode = causal ? 1 : 0;
   const int npages = batch > 0 ? kv[batch] : 0;
@@ -666,7 +664,7 @@ int fe_attn_plan_prepare(fe_attn_plan* p, const int32_t* qo, const int32_t* kv, 
   if (cap != hipStreamCaptureStatusNone)
     return fail(FE_EINVAL, "prepare_plan: the stream is capturing a graph; prepare outside the capture and "
                            "capture only the attention calls");
-  rc = build_plan(L.sh, qo, kv, pages, last, batch, rows, bp, err, short_waves(L.sh));
+  rc = build_plan(L.sh, qo, kv, pages, last, batch, rows, bp, err, short_waves(L.sh), true);
   if (rc != FE_OK) return fail(rc, err);
   int nc = bp.decode_nc;
   int graph_nc = p->graph_nc, graph_tile = L.graph_tile;

@@ -164,6 +164,7 @@ bool cut_tile_stream(const std::vector<SeqInfo>& seqs, int G, int hkv, bool caus
   if (rows > slot_budget) return false;
 
   ModeLists out;
+  out.tile_rows = qr;
   out.partial_rows = (int)rows;
   for (size_t i = 0; i < ch.size(); ++i)
     if (base[i] >= 0)
@@ -290,6 +291,58 @@ bool plan_short(const PlanShape& sh, const int32_t* pages, int waves, BuiltPlan&
   return true;
 }
 
+// A small amount of tile work as items of half a tile's columns over their
+// whole visible range, or false (leaving `ml` alone) where full-width items,
+// split over the tokens and merged, are faster.
+//
+// While workgroups do not fill the chip an item's time is its chain of tiles:
+// about 7 us for the launch and the first tile, then 0.6-0.8 us a tile at 64
+// columns against 0.9-1.4 at 128; splitting the tokens costs the merge launch
+// and, however small the call, 15 us.  So short chains are not split, and
+// longer ones only need enough items (n) for their total to outweigh the
+// split plan's start.  Measured on the MI355X, us a call, this form against
+// full-width items, split where that list splits them:
+//   * up to 8 tiles: 8.2 / 10.9 (256 tokens, 16/8 heads), 12.5 / 19.6 (512,
+//     32/8), 15.5 / 21.9 (4 x 512, 16/8); at n = 1024 only equal (18.6 / 18.1).
+//   * up to 13 tiles from n = 12 tiles on: 16.0 / 19.5 (777 tokens, 16/8: n =
+//     200), 22.8 / 29.9 (4 x 256 over 500, 32/8).
+//   * longer ones from n = 16 tiles on: 20.5 / 21.3 (1024, 16/8: 16 tiles, n =
+//     256), 23.7 / 28.3 (1024, 32/8), 34.9 / 47.6 (1500, 32/8), 44.1 / 45.9
+//     (1024 over 1000 cached, 32/8: 32 tiles, n = 512); below it 21.5 / 15.2
+//     (64 over 1000, 16/8: n = 16), 27.4 / 22.3 (512 over 1000, 16/8).
+//   * 9 and 10 tiles gain where the items are half as wide, 13.8 / 15.9 (4 x
+//     64 over 500, 16/8), not where they were 64 columns already, 12.4 / 11.4
+//     (16 rows over 500, 32/8).
+//   * without the causal mask every item is a whole chain: 39.9 / 37.4 (32 x
+//     16 rows over 1000, 40/8: 16 tiles), 21.9 / 28.4 over 500.
+bool plan_small_tiles(const PlanShape& sh, bool causal, const BuiltPlan& bp, ModeLists& ml) {
+  constexpr int kMaxItems = 768;
+  const int G = sh.hq / sh.hkv;
+  const int qr = kTileCols / 2 / G;  // query rows per item
+  if (qr < 1) return false;
+  std::vector<WorkItem> items;
+  int longest = 0;
+  bool halved = false;
+  for (int b = 0; b < (int)bp.seqs.size(); ++b) {
+    const SeqInfo& s = bp.seqs[b];
+    if (s.qlen * G <= kDecodeCols) continue;
+    halved = halved || s.qlen > qr;
+    for (int i0 = 0; i0 < s.qlen; i0 += qr) {
+      const int nq = std::min(qr, s.qlen - i0);
+      const int extent = causal ? std::min(s.len, s.len - s.qlen + i0 + nq) : s.len;
+      const int tiles = ceil_div(extent, kTileTokens);
+      longest = std::max(longest, tiles);
+      if (longest > (causal ? 32 : 13) || items.size() + (size_t)sh.hkv > kMaxItems) return false;
+      for (int h = 0; h < sh.hkv; ++h) items.push_back(WorkItem{b, s.qo + i0, nq, h, 0, extent, -1, tiles});
+    }
+  }
+  if (longest > (halved ? 10 : 8) && (int)items.size() < (longest <= 13 ? 12 : 16) * longest) return false;
+  ml.tile = std::move(items);
+  ml.tile_rows = qr;
+  assign_shares(ml.tile, sh.tile_slots, ml.tile_off, sh.num_cus);
+  return true;
+}
+
 }  // namespace
 
 int validate_shape(const PlanShape& sh, std::string& err) {
@@ -317,7 +370,8 @@ int validate_shape(const PlanShape& sh, std::string& err) {
 }
 
 static int build_plan_impl(const PlanShape& sh, const int32_t* qo, const int32_t* kv, const int32_t* pages,
-               const int32_t* last, int batch, int rows, BuiltPlan& out, std::string& err, int short_waves) {
+               const int32_t* last, int batch, int rows, BuiltPlan& out, std::string& err, int short_waves,
+               bool small_tiles) {
   int rc = validate_shape(sh, err);
   if (rc != FE_OK) return rc;
   if (batch < 0 || rows < 0) {
@@ -500,6 +554,7 @@ static int build_plan_impl(const PlanShape& sh, const int32_t* qo, const int32_t
   for (int causal = 0; causal < 2; ++causal) {
     ModeLists& ml = out.mode[causal];
     ml.partial_rows = out.decode_partials;
+    ml.tile_rows = qr;
     // (q tile, kv head) pairs before splitting, to size the split factor.
     int64_t pairs = 0;
     for (int b = 0; b < batch; ++b) {
@@ -507,6 +562,7 @@ static int build_plan_impl(const PlanShape& sh, const int32_t* qo, const int32_t
       if (s.qlen * G > kDecodeCols) pairs += (int64_t)ceil_div(s.qlen, qr) * sh.hkv;
     }
     if (pairs == 0) continue;
+    if (small_tiles && plan_small_tiles(sh, causal != 0, out, ml)) continue;
     // Aim for about 8 items per compute unit (2 resident workgroups, several
     // rounds in longest-first order); never split below 256 tokens.
     int want = (int)std::max<int64_t>(1, ((int64_t)sh.num_cus * 8 + pairs - 1) / pairs);
@@ -579,9 +635,10 @@ static int build_plan_impl(const PlanShape& sh, const int32_t* qo, const int32_t
 }
 
 int build_plan(const PlanShape& sh, const int32_t* qo, const int32_t* kv, const int32_t* pages,
-               const int32_t* last, int batch, int rows, BuiltPlan& out, std::string& err, int short_waves) {
+               const int32_t* last, int batch, int rows, BuiltPlan& out, std::string& err, int short_waves,
+               bool small_tiles) {
   try {
-    return build_plan_impl(sh, qo, kv, pages, last, batch, rows, out, err, short_waves);
+    return build_plan_impl(sh, qo, kv, pages, last, batch, rows, out, err, short_waves, small_tiles);
   } catch (const std::bad_alloc&) {
     err = "out of host memory while building the work lists";
     return FE_ENOMEM;

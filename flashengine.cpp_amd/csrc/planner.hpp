@@ -29,6 +29,7 @@ struct PlanShape {
 struct ModeLists {
   std::vector<WorkItem> tile;            // grouped by share: share k = [tile_off[k], tile_off[k+1])
   std::vector<int32_t> tile_off;         // CSR over shares (one share per tile workgroup)
+  int tile_rows = 0;                     // query rows of a tile item at most
   std::vector<MergeRow> merge;
   int partial_rows = 0;  // decode partials followed by this mode's tile partials
 };
@@ -62,8 +63,10 @@ int validate_shape(const PlanShape& sh, std::string& err);
 //
 // short_waves > 0: a batch of decode sequences that is faster so is planned
 // as short-context items for workgroups of that many wavefronts
-// (`shorts`) instead of decode shares.
+// (`shorts`) instead of decode shares.  small_tiles: tile work that is faster
+// so is planned as unsplit items of half a tile's columns.
 int build_plan(const PlanShape& sh, const int32_t* qo, const int32_t* kv, const int32_t* pages,
-               const int32_t* last, int batch, int rows, BuiltPlan& out, std::string& err, int short_waves = 0);
+               const int32_t* last, int batch, int rows, BuiltPlan& out, std::string& err, int short_waves = 0,
+               bool small_tiles = false);
 
 }  // namespace feattn

@@ -150,11 +150,61 @@ static bool check(const Case& c, int waves, int& taken) {
   return true;
 }
 
+// Plans with small_tiles: where a mode's tile list is not the ordinary one,
+// its items are unsplit, at most 64 columns wide, cover every row of the tile
+// sequences once per kv head over all the tokens it sees, and its shares
+// cover the list.
+static bool check_tiles(const Case& c, int& taken) {
+  BuiltPlan bp, plain;
+  std::string err;
+  CHECK(build_plan(c.sh, c.qo.data(), c.kv.data(), c.pages.data(), c.last.data(), c.batch, c.rows, bp, err, 0, true) ==
+        FE_OK);
+  CHECK(build_plan(c.sh, c.qo.data(), c.kv.data(), c.pages.data(), c.last.data(), c.batch, c.rows, plain, err) ==
+        FE_OK);
+  const int G = c.sh.hq / c.sh.hkv;
+  CHECK(bp.decode.size() == plain.decode.size() && bp.decode_partials == plain.decode_partials);
+  for (int causal = 0; causal < 2; ++causal) {
+    const ModeLists& ml = bp.mode[causal];
+    if (ml.tile.empty()) continue;
+    CHECK(ml.tile_rows >= 1 && ml.tile_rows * G <= kTileCols);
+    for (const WorkItem& w : ml.tile) CHECK(w.nq <= ml.tile_rows);
+    if (ml.tile_rows == plain.mode[causal].tile_rows) {
+      CHECK(ml.tile.size() == plain.mode[causal].tile.size() && ml.tile_off == plain.mode[causal].tile_off);
+      continue;
+    }
+    ++taken;
+    CHECK(ml.tile_rows == kTileCols / 2 / G && ml.partial_rows == bp.decode_partials);
+    CHECK(ml.merge.size() == bp.decode_merge.size());
+    CHECK(!ml.tile_off.empty() && ml.tile_off.front() == 0 && ml.tile_off.back() == (int)ml.tile.size());
+    CHECK((int)ml.tile_off.size() - 1 <= c.sh.tile_slots);
+    std::map<std::pair<int, int>, int> seen;  // (row, kv head) -> end of its tokens
+    for (const WorkItem& w : ml.tile) {
+      CHECK(w.part == -1 && w.t0 == 0 && w.nq >= 1);
+      const SeqInfo& s = bp.seqs[w.seq];
+      CHECK(w.q0 >= s.qo && w.q0 + w.nq <= s.qo + s.qlen && w.t1 <= s.len);
+      for (int r = 0; r < w.nq; ++r) CHECK(seen.emplace(std::make_pair(w.q0 + r, w.kvh), w.t1).second);
+    }
+    size_t want = 0;
+    for (const SeqInfo& s : bp.seqs) {
+      if (s.qlen * G <= kDecodeCols) continue;
+      for (int i = 0; i < s.qlen; ++i)
+        for (int h = 0; h < c.sh.hkv; ++h, ++want)
+          CHECK((seen[{s.qo + i, h}] >= (causal ? s.len - s.qlen + i + 1 : s.len)));
+    }
+    CHECK(want == seen.size());
+  }
+  return true;
+}
+
 int main() {
   std::mt19937 rng(7);
-  int taken = 0, n = 0;
+  int taken = 0, n = 0, tiles = 0;
   for (int i = 0; i < 3000; ++i) {
     const Case c = make(rng);
+    if (!check_tiles(c, tiles)) {
+      printf("batch %d, small tiles\n", i);
+      return 1;
+    }
     for (int waves : {4, 8}) {
       ++n;
       if (!check(c, waves, taken)) {
@@ -163,6 +213,6 @@ int main() {
       }
     }
   }
-  printf("%d plans, %d short\n", n, taken);
-  return g_fail || taken < n / 20 || taken == n;
+  printf("%d plans, %d short, %d small tile lists\n", n, taken, tiles);
+  return g_fail || taken < n / 20 || taken == n || tiles < 100;
 }

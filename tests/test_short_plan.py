@@ -1,5 +1,5 @@
-"""Short-context plans (planner.cpp: plan_short): the item lists over random
-batches, built with AddressSanitizer and UndefinedBehaviorSanitizer
+"""Plans of small calls (planner.cpp: plan_short, plan_small_tiles): the item
+lists over random batches, built with AddressSanitizer and UndefinedBehaviorSanitizer
 (tests/cpp/short_check.cpp), and on the GPU the kernel's edges against the
 oracle."""
 import os
@@ -92,3 +92,32 @@ def test_short_kernel_edges(dev, hq, hkv, rows, page, dtype, causal):
             assert torch.equal(out, got[0][0]) and torch.equal(lse, got[0][1])
     plan.close()
     graph_plan.close()
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("hq,hkv,starts,qlens", [
+    (16, 8, [0], [17]), (16, 8, [0, 0, 0], [32, 33, 65]), (16, 8, [0], [777]), (32, 8, [0, 31], [15, 17]),
+    (32, 8, [448, 0], [64, 512]), (32, 8, [449], [64]), (32, 4, [500, 100], [9, 40]), (40, 8, [300, 7], [12, 13]),
+    (64, 1, [0, 90], [5, 70]), (32, 8, [100, 700, 0], [48, 1, 3]), (32, 8, [0], [1100])])
+@pytest.mark.parametrize("dtype,causal", [("bf16", True), ("f16", False)])
+def test_small_tile_items(dev, hq, hkv, starts, qlens, dtype, causal):
+    """Chunks at the edges of the 64-column items and of the rule that makes
+    them, some beside decode rows, against the oracle (tolerance of the other
+    attention tests); a graph plan gives the same bits."""
+    b = W.make_batch(hq, hkv, starts=starts, qlens=qlens, seed=11, extra_pages=2)
+    q, kc, vc = W.make_tensors(b, seed=5, dtype=dtype)
+    want, want_lse = A.run(b, q, kc, vc, causal)
+    q, kc, vc = q.to(dev), kc.to(dev), vc.to(dev)
+    got = []
+    for graph in (False, True):
+        plan = feattn.Plan(hq, hkv, 128, 16, b.batch, b.max_pages(), dtype == "bf16", b.blocks)
+        plan.prepare(b.qo, b.kv, b.pages, b.last, b.batch, b.rows, graph=graph)
+        out = torch.full_like(q, float("nan"))
+        lse = torch.full((b.rows, hq), float("nan"), device=dev)
+        plan.run(q, kc, vc, out, causal=causal, lse=lse)
+        torch.cuda.synchronize()
+        plan.close()
+        torch.testing.assert_close(out.float().cpu(), want.float(), atol=1e-2, rtol=1e-2)
+        torch.testing.assert_close(lse.cpu(), want_lse, atol=1e-3, rtol=0)
+        got.append((out, lse))
+    assert torch.equal(got[0][0], got[1][0]) and torch.equal(got[0][1], got[1][1])
