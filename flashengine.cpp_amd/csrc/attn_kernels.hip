@@ -7,7 +7,7 @@
 // (scores pre-multiplied by log2(e)/sqrt(128)); log-sum-exp is kept in log2
 // units internally and converted to natural log on output.
 //
-// Three kernels:
+// Kernels:
 //  * attn_decode_kernel: persistent; each wavefront walks one share of the
 //    decode token stream for one kv head (pieces of <= 16 (query row, head)
 //    columns: decode rows x GQA heads along the MFMA N dimension), copying
@@ -17,8 +17,12 @@
 //    LDS; each wavefront owns 16 or 32 (query row, head) columns and
 //    computes S^T = K Q^T and O^T = V^T P^T on the bf16/fp16 MFMA with fp32
 //    accumulation (chunked prefill, DFlash blocks, verify rows).
-//  * attn_merge_kernel: combines split-KV partials by their log-sum-exp, one
-//    wavefront per (query row, head) with a batch of splits in flight.
+//  * attn_short_kernel (attn_short.hpp): short decode batches, one workgroup
+//    per item with its tokens divided among the wavefronts; graph launches
+//    reach it through attn_decode_kernel<..., true>.
+//  * attn_merge_kernel: combines split-KV partials by their log-sum-exp, a
+//    wavefront or a workgroup per (query row, pair of heads) with batches of
+//    splits in flight.
 // and stage_copy_kernel, which moves a prepared plan's metadata from pinned
 // host memory into its device arena on the caller's stream.
 #include <algorithm>

@@ -71,8 +71,9 @@ int fe_attn_plan_destroy(fe_attn_plan* plan);
  * lists and copies them to the plan's device buffers on `stream` (one small
  * kernel on `stream` reads the plan's pinned staging memory; the call waits
  * for the previous prepare's transfer before reusing that memory).
- * `graph` != 0 pins the launch grids to the plan capacity so that a graph
- * captured once replays correctly after later prepares.  `stream` must be
+ * `graph` != 0 makes the launches independent of this batch's lists (grids
+ * that cover or loop over any later prepare's) so that a graph captured once
+ * replays correctly after later prepares.  `stream` must be
  * on the device that was current when the plan was created (FE_EDEVICE
  * otherwise), here and in fe_attn_run. */
 int fe_attn_plan_prepare(fe_attn_plan* plan, const int32_t* qo,
@@ -155,8 +156,9 @@ int fe_attn_run_noalloc(const void* q, const void* k_cache, const void* v_cache,
 const char* fe_attn_last_error(void);
 
 /* Host-only planner introspection (no device needed): runs the same
- * validation and work-list construction as fe_attn_plan_prepare and reports
- * the counts.  Used by tests and by the benchmark to report the split-KV
+ * validation as fe_attn_plan_prepare and reports the counts of the general
+ * plan (shares and full-width tile items; prepare plans small calls in other
+ * forms where those are faster).  Used by tests and by the benchmark to report the split-KV
  * layout.  counts_out[0..3] = decode items, tile items, merge rows,
  * partial rows. */
 int fe_attn_plan_describe(int hq, int hkv, int dim, int page, int max_batch,
