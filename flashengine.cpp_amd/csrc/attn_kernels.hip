@@ -753,18 +753,27 @@ __device__ __forceinline__ MergeRow ldc_merge(const MergeRow* rows, int i) {
 template <bool BF16, int BATCH>
 __device__ __forceinline__ void merge_fold(const MergeArgs& a, const MergeRow& mr, int head, int d, int sp0,
                                            MergeState& s) {
+  size_t slot[BATCH];
   float l[BATCH];
   u32x2 rv[BATCH];  // four 16-bit partial values
-  // Past the last split the loads repeat it (a cache hit) and its weight is
-  // zero: a branch around each load lets the compiler move the 16-bit
-  // conversions into it, behind a wait per load (verify rows in fp16: the
-  // call took 66.9 us so, 63.6 without).
+  // Past the last split the loads repeat it (a cache hit); what they brought
+  // is replaced by zero with weight zero (a repeated infinity times zero would
+  // be NaN).  A branch around each load lets the compiler move the 16-bit
+  // conversions into it, behind a wait per load (verify rows in fp16: the call
+  // took 66.9 us so, 63.6 without).  The scheduling barriers keep all loads in
+  // flight together, the log-sum-exps first, and the weights before the first
+  // wait for a value (without them the values' loads sink below the wait for
+  // the log-sum-exps, or their conversions rise above it: 0.3 us a call).
 #pragma unroll
   for (int u = 0; u < BATCH; ++u) {
-    const size_t slot = (size_t)(mr.part + min(sp0 + u, mr.nsplit - 1) * mr.stride);
-    l[u] = a.part_lse[slot * a.hq + head];
-    rv[u] = *reinterpret_cast<const u32x2*>(a.part_o + (slot * a.hq + head) * kHeadDim + d);
+    slot[u] = (size_t)(mr.part + min(sp0 + u, mr.nsplit - 1) * mr.stride) * a.hq + head;
+    l[u] = a.part_lse[slot[u]];
   }
+  __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+  for (int u = 0; u < BATCH; ++u)
+    rv[u] = *reinterpret_cast<const u32x2*>(a.part_o + slot[u] * kHeadDim + d);
+  __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
   for (int u = 0; u < BATCH; ++u)
     if (sp0 + u >= mr.nsplit) l[u] = kNegInf;
@@ -776,12 +785,15 @@ __device__ __forceinline__ void merge_fold(const MergeArgs& a, const MergeRow& m
   s.wsum *= sc;
   s.acc *= sc;
 #pragma unroll
+  for (int u = 0; u < BATCH; ++u) l[u] = fast_exp2(l[u] - mu);
+  __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
   for (int u = 0; u < BATCH; ++u) {
-    const float wt = fast_exp2(l[u] - mu);
+    rv[u] &= sp0 + u < mr.nsplit ? ~0u : 0u;
     const f32x4 v = {lo_f32<BF16>(rv[u][0]), hi_f32<BF16>(rv[u][0]), lo_f32<BF16>(rv[u][1]),
                      hi_f32<BF16>(rv[u][1])};
-    s.wsum += wt;
-    s.acc += wt * v;
+    s.wsum += l[u];
+    s.acc += l[u] * v;
   }
   s.m = bm;
 }

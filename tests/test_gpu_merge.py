@@ -42,3 +42,34 @@ def test_split_counts(dev, dtype, rows):
         assert torch.equal(got[0][0], got[1][0]) and torch.equal(got[0][1], got[1][1])
     plan.close()
     graph_plan.close()
+
+
+@pytest.mark.parametrize("dtype", ["bf16", "f16"])
+def test_infinite_values_stay_infinite(dev, dtype):
+    """Infinite V entries in a row's first and last split, for split counts
+    around and between the batches of both merge forms: every weight is
+    positive, so the output is that infinity, exactly the elements of the
+    oracle's that are; the others are within the tolerance."""
+    hq = hkv = 5  # shares of 64 tokens: ceil(tokens / 64) splits
+    plan = feattn.Plan(hq, hkv, 128, 16, 1, 300, dtype == "bf16", 600)
+    graph_plan = feattn.Plan(hq, hkv, 128, 16, 1, 300, dtype == "bf16", 600)
+    for splits in (2, 3, 4, 5, 7, 8, 9, 16, 17, 33, 65):
+        n = 64 * splits - 5
+        b = W.make_batch(hq, hkv, starts=[n - 1], qlens=[1], seed=splits, pool=600)
+        q, kc, vc = W.make_tensors(b, seed=4, dtype=dtype)
+        for tok, head, dim, sign in ((0, 0, 3, 1), (n - 1, 1, 17, 1), (n - 2, 4, 127, -1)):
+            vc[b.tables[0][tok // 16], tok % 16, head, dim] = sign * float("inf")
+        want, _ = A.run(b, q, kc, vc, True)
+        inf = torch.isinf(want.float())
+        assert int(inf.sum()) == 3 and not torch.isnan(want.float()).any()
+        q, kc, vc = q.to(dev), kc.to(dev), vc.to(dev)
+        for p, graph in ((plan, False), (graph_plan, True)):
+            p.prepare(b.qo, b.kv, b.pages, b.last, b.batch, b.rows, graph=graph)
+            out = torch.full_like(q, float("nan"))
+            p.run(q, kc, vc, out, causal=True)
+            torch.cuda.synchronize()
+            out = out.float().cpu()
+            assert torch.equal(out[inf], want.float()[inf]), splits
+            torch.testing.assert_close(out[~inf], want.float()[~inf], atol=1e-2, rtol=1e-2)
+    plan.close()
+    graph_plan.close()
