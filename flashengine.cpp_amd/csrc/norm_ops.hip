@@ -322,11 +322,14 @@ __global__ __launch_bounds__(256) void norm_rope_append_kernel(
 // ---------------------------------------------------------------------------
 __device__ __forceinline__ float silu_any(float x) { return __fdiv_rn(x, __fadd_rn(1.f, expf(-x))); }
 
-// The same for |x| < kSiluFast, where neither the exponential nor the
-// quotient can leave the normal range, so that no scaling and no special
-// case is needed.  exp(-x) = 2^n 2^f with n the nearest integer to -x
+// The same for |x| < kSiluFast, where neither the exponential nor 1 + exp(-x)
+// nor its reciprocal can leave the normal range, so that no scaling and no
+// special case is needed.  exp(-x) = 2^n 2^f with n the nearest integer to -x
 // log2(e) and f the rest, taken with log2(e) in two floats.  The quotient is
-// the reciprocal estimate's, corrected once by its exact residual.
+// the reciprocal estimate's, corrected once by its residual; it is subnormal
+// only for |x| < 2^-125 (bf16), where 1 + exp(-x) is 2 and quotient and
+// residual are exact.  The residual step turns a quotient of -0 into +0, so
+// the sign, which is x's everywhere, is put back.
 constexpr float kSiluFast = 80.f;
 __device__ __forceinline__ float silu_fast(float x) {
   constexpr float kL2e = 1.44269502162933349609375f;  // log2(e) rounded to float
@@ -337,7 +340,7 @@ __device__ __forceinline__ float silu_fast(float x) {
   const float d = __fadd_rn(1.f, e);
   const float r = __builtin_amdgcn_rcpf(d);
   const float q = __fmul_rn(x, r);
-  return __builtin_fmaf(__builtin_fmaf(-q, d, x), r, q);
+  return __builtin_copysignf(__builtin_fmaf(__builtin_fmaf(-q, d, x), r, q), x);
 }
 
 // n / d for n < 2^31 by a multiplication: mul = floor(2^(31 + l) / d) + 1 with

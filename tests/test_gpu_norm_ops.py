@@ -292,8 +292,8 @@ def test_silu_mul_within_one_step(dev, bf16):
 
 
 def silu_close(got, want, bf16):
-    """One rounding step of the 16-bit type; NaN for NaN, infinities and the
-    sign of results that underflow equal."""
+    """One rounding step of the 16-bit type; NaN for NaN, infinities and every
+    sign (of zeros and of results that underflow too) equal."""
     a, b = R.to_f32(got, bf16).astype(np.float64), R.to_f32(want, bf16).astype(np.float64)
     assert np.array_equal(np.isnan(a), np.isnan(b))
     if bf16:
@@ -301,6 +301,7 @@ def silu_close(got, want, bf16):
     inf = np.isinf(a) | np.isinf(b)
     assert np.array_equal(a[inf], b[inf])
     ok = ~(np.isnan(a) | inf)
+    assert np.array_equal(np.signbit(a[~np.isnan(a)]), np.signbit(b[~np.isnan(b)]))
     # a result below 2^-126 has float32's own absolute spacing behind it
     step = np.maximum(np.abs(a), np.abs(b))[ok] * (2.0 ** -7 if bf16 else 2.0 ** -10) + (2.0 ** -133 if bf16
                                                                                         else 2.0 ** -24)
