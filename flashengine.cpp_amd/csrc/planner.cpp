@@ -296,47 +296,74 @@ bool plan_short(const PlanShape& sh, const int32_t* pages, int waves, BuiltPlan&
 // split over the tokens and merged, are faster.
 //
 // While workgroups do not fill the chip an item's time is its chain of tiles:
-// about 7 us for the launch and the first tile, then 0.6-0.8 us a tile at 64
-// columns against 0.9-1.4 at 128; splitting the tokens costs the merge launch
-// and, however small the call, 15 us.  So short chains are not split, and
-// longer ones only need enough items (n) for their total to outweigh the
-// split plan's start.  Measured on the MI355X, us a call, this form against
-// full-width items, split where that list splits them:
-//   * up to 8 tiles: 8.2 / 10.9 (256 tokens, 16/8 heads), 12.5 / 19.6 (512,
-//     32/8), 15.5 / 21.9 (4 x 512, 16/8); at n = 1024 only equal (18.6 / 18.1).
-//   * up to 13 tiles from n = 12 tiles on: 16.0 / 19.5 (777 tokens, 16/8: n =
-//     200), 22.8 / 29.9 (4 x 256 over 500, 32/8).
-//   * longer ones from n = 16 tiles on: 20.5 / 21.3 (1024, 16/8: 16 tiles, n =
-//     256), 23.7 / 28.3 (1024, 32/8), 34.9 / 47.6 (1500, 32/8), 44.1 / 45.9
-//     (1024 over 1000 cached, 32/8: 32 tiles, n = 512); below it 21.5 / 15.2
-//     (64 over 1000, 16/8: n = 16), 27.4 / 22.3 (512 over 1000, 16/8).
-//   * 9 and 10 tiles gain where the items are half as wide, 13.8 / 15.9 (4 x
-//     64 over 500, 16/8), not where they were 64 columns already, 12.4 / 11.4
-//     (16 rows over 500, 32/8).
-//   * without the causal mask every item is a whole chain: 39.9 / 37.4 (32 x
-//     16 rows over 1000, 40/8: 16 tiles), 21.9 / 28.4 over 500.
+// about 4.4 us for the launch and the first tile, then 0.93 us a tile of 64
+// tokens, and little for the other items (0.2 us per 64 x 64 block of the
+// call's whole area on each compute unit).  Splitting the tokens costs the
+// merge launch, about 14 us however small the call, and 0.8 us per block of
+// area.  So unsplit items win below a line in the longest chain that rises
+// with the area, and falls where many sequences' cached K/V, which narrower
+// items read twice, stand against it (a tile for every 25 KB on each compute
+// unit).  All are taken exactly, not in whole tiles or items, so that
+// neighbouring lengths of a prompt get the same plan.  Fitted over 4087 timed
+// batches (12 head counts, prompts, chunks over a prefix, 16-row blocks, eager
+// and in graphs; MI355X): 13 of them are more than 3 % slower than with
+// full-width items, 1.5 us at most.  us a call, this form against those:
+//   * no sequence of 512 tokens: the other list does not split either, and
+//     half-width items only halve a tile's work.  12.9 / 17.3 (4 x 208 over
+//     300, 16/8 heads, area 5.1), 16.0 / 18.5 (32/8, 10.3), 16.4 / 17.0 (16 x
+//     48 over 298, 40/8, 9.5); from area 11 on slower, 21.0 / 19.0 (4 x 194
+//     over 300, 40/8, 11.8), 30.4 / 25.2 (64 x 16 over 456, 32/4, all visible,
+//     14.8).
+//   * longer ones at little area: 15.6 / 18.0 (256 over 500, 16/8: 12 tiles,
+//     area 2.5), 20.2 / 15.2 (64 over 1000, 16/8: 17 tiles, 1.0).
+//   * prompts, 16/8: 15.2 / 18.9 (704 tokens), 17.2 / 19.7 (848), 18.3 / 19.8
+//     (896, in a graph 21.9 / 21.7), 20.1 / 20.5 (992, in a graph 23.7 / 22.3),
+//     25.8 / 24.9 (1328); 32/8: 23.2 / 27.5 (1024, area 16).
+//   * 16-row blocks, all visible: 36.8 / 29.7 (64 over 1146, 12/2 heads, 290 KB
+//     of K/V per compute unit), 33.2 / 28.4 (16 over 1043, 40/8, 265 KB).
+//   * items that are whole columns already (at most 64 in a sequence) gain
+//     only the merge: the line lies 3.5 tiles lower.  17.5 / 21.6 (32 x 16
+//     over 250 to 500, 32/8: 8 tiles, area 6), 18.1 / 14.7 (4 x 16 over up to
+//     750: 12 tiles, 1.3).
+//   * past an area of 40 the chip is full and the form no longer matters or
+//     loses: 24.3 / 31.8 at 20 (1024 tokens, 40/8), 52.8 / 51.1 at 51 (912 over
+//     1000), 94.2 / 70.1 at 71 (64 x 16 over 2253, 32/4, all visible).
 bool plan_small_tiles(const PlanShape& sh, bool causal, const BuiltPlan& bp, ModeLists& ml) {
-  constexpr int kMaxItems = 768;
+  constexpr int64_t kMaxItems = 768;  // (a bound on the list; fuller chips are past the area's)
   const int G = sh.hq / sh.hkv;
   const int qr = kTileCols / 2 / G;  // query rows per item
   if (qr < 1) return false;
-  std::vector<WorkItem> items;
+  int64_t n_items = 0, visible = 0, cached = 0;  // visible: (query row, token) pairs
   int longest = 0;
   bool halved = false;
+  for (const SeqInfo& s : bp.seqs) {
+    if (s.qlen * G <= kDecodeCols) continue;
+    n_items += (int64_t)ceil_div(s.qlen, qr) * sh.hkv;
+    const int64_t full = (int64_t)s.qlen * s.len;
+    visible += causal ? full - (int64_t)s.qlen * (s.qlen - 1) / 2 : full;
+    cached += s.len - s.qlen;
+    longest = std::max(longest, s.len);
+    halved = halved || s.qlen > qr;
+  }
+  if (n_items > kMaxItems) return false;
+  const double area = (double)visible * sh.hq / ((double)kTileTokens * kTileTokens * sh.num_cus);
+  const double cached_kb = (double)cached * sh.hkv * (2 * kHeadDim * 2) / (1024.0 * sh.num_cus);
+  if (longest < 512 ? area > 11.0
+                    : area > 40.0 || (double)longest / kTileTokens >
+                                         (halved ? 10.5 : 7.0) + 0.62 * area - 0.04 * cached_kb)
+    return false;
+  std::vector<WorkItem> items;
+  items.reserve((size_t)n_items);
   for (int b = 0; b < (int)bp.seqs.size(); ++b) {
     const SeqInfo& s = bp.seqs[b];
     if (s.qlen * G <= kDecodeCols) continue;
-    halved = halved || s.qlen > qr;
     for (int i0 = 0; i0 < s.qlen; i0 += qr) {
       const int nq = std::min(qr, s.qlen - i0);
       const int extent = causal ? std::min(s.len, s.len - s.qlen + i0 + nq) : s.len;
-      const int tiles = ceil_div(extent, kTileTokens);
-      longest = std::max(longest, tiles);
-      if (longest > (causal ? 32 : 13) || items.size() + (size_t)sh.hkv > kMaxItems) return false;
-      for (int h = 0; h < sh.hkv; ++h) items.push_back(WorkItem{b, s.qo + i0, nq, h, 0, extent, -1, tiles});
+      for (int h = 0; h < sh.hkv; ++h)
+        items.push_back(WorkItem{b, s.qo + i0, nq, h, 0, extent, -1, ceil_div(extent, kTileTokens)});
     }
   }
-  if (longest > (halved ? 10 : 8) && (int)items.size() < (longest <= 13 ? 12 : 16) * longest) return false;
   ml.tile = std::move(items);
   ml.tile_rows = qr;
   assign_shares(ml.tile, sh.tile_slots, ml.tile_off, sh.num_cus);

@@ -196,7 +196,45 @@ static bool check_tiles(const Case& c, int& taken) {
   return true;
 }
 
+// One causal prompt of growing length, nothing cached: the tile list takes the
+// small form from the first length on and changes to the ordinary one at most
+// once.  (ordinary: the length from which it does.)
+static bool check_prompts(int hq, int hkv, int& ordinary) {
+  const int G = hq / hkv, most = 3000;
+  Case c;
+  c.sh.hq = hq;
+  c.sh.hkv = hkv;
+  c.sh.dim = 128;
+  c.sh.page = 16;
+  c.sh.max_batch = 1;
+  c.sh.max_pages = most / 16 + 2;
+  c.sh.blocks = most;
+  c.sh.partial_cap = 8192;
+  for (int i = 0; i <= most / 16; ++i) c.pages.push_back(i);
+  ordinary = 0;
+  for (int n = kDecodeCols / G + 1; n <= most; n += n < 1500 ? 3 : 7) {
+    const int np = (n + 15) / 16;
+    const int32_t qo[2] = {0, n}, kv[2] = {0, np}, last[1] = {n - 16 * (np - 1)};
+    BuiltPlan bp;
+    std::string err;
+    CHECK(build_plan(c.sh, qo, kv, c.pages.data(), last, 1, n, bp, err, 0, true) == FE_OK);
+    const bool small = bp.mode[1].tile_rows == kTileCols / 2 / G;
+    if (!small && ordinary == 0) ordinary = n;
+    CHECK(!small || ordinary == 0);
+  }
+  return true;
+}
+
 int main() {
+  static const int heads[][2] = {{4, 1},  {8, 2},  {8, 8},  {12, 2}, {16, 2}, {16, 8},
+                                 {28, 4}, {32, 4}, {32, 8}, {40, 8}, {64, 4}, {64, 8}};
+  for (const auto& h : heads) {
+    int at = 0;
+    if (!check_prompts(h[0], h[1], at) || at < 300) {
+      printf("prompts, %d/%d heads: ordinary from %d tokens\n", h[0], h[1], at);
+      return 1;
+    }
+  }
   std::mt19937 rng(7);
   int taken = 0, n = 0, tiles = 0;
   for (int i = 0; i < 3000; ++i) {

@@ -98,7 +98,8 @@ def test_short_kernel_edges(dev, hq, hkv, rows, page, dtype, causal):
 @pytest.mark.parametrize("hq,hkv,starts,qlens", [
     (16, 8, [0], [17]), (16, 8, [0, 0, 0], [32, 33, 65]), (16, 8, [0], [777]), (32, 8, [0, 31], [15, 17]),
     (32, 8, [448, 0], [64, 512]), (32, 8, [449], [64]), (32, 4, [500, 100], [9, 40]), (40, 8, [300, 7], [12, 13]),
-    (64, 1, [0, 90], [5, 70]), (32, 8, [100, 700, 0], [48, 1, 3]), (32, 8, [0], [1100])])
+    (64, 1, [0, 90], [5, 70]), (32, 8, [100, 700, 0], [48, 1, 3]), (32, 8, [0], [1100]), (16, 8, [0], [912]),
+    (16, 8, [0], [960]), (40, 8, [300] * 4, [180] * 4), (40, 8, [300] * 4, [194] * 4)])
 @pytest.mark.parametrize("dtype,causal", [("bf16", True), ("f16", False)])
 def test_small_tile_items(dev, hq, hkv, starts, qlens, dtype, causal):
     """Chunks at the edges of the 64-column items and of the rule that makes
