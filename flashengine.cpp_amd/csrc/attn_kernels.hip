@@ -131,7 +131,7 @@ __global__ __launch_bounds__(64 * WAVES, ANY ? 2 : 1) void attn_decode_kernel(At
   const ShareStart rec = ldc_share(a.shares, ANY ? min(share, a.n_share_cap - 1) : share);
   if constexpr (ANY) {
     if (rec.n_short > 0) {
-      short_items<BF16, WAVES, NCB>(a, causal, rec.n_short, dsm);
+      short_items<BF16, WAVES, NCB, false>(a, causal, rec.n_short, dsm);
       return;
     }
     if (share >= a.n_share_cap) return;
@@ -891,7 +891,7 @@ int decode_wg_waves(int hkv) {
 template <bool BF16, int WAVES, int NCB>
 __global__ __launch_bounds__(64 * WAVES, 2) void attn_short_kernel(AttnArgs a, int causal) {
   extern __shared__ __attribute__((aligned(16))) uint8_t dsm[];
-  short_items<BF16, WAVES, NCB>(a, causal, a.n_short, dsm);
+  short_items<BF16, WAVES, NCB, true>(a, causal, 1, dsm);
 }
 
 enum class DecodeKind { Shares, Short, Any };
@@ -907,7 +907,9 @@ static hipError_t decode_launch(const AttnArgs& a, int causal, int grid, hipStre
   static std::atomic<uint64_t> lds_ok{0};
   const hipError_t e = allow_lds((const void*)fn, lds, lds_ok);
   if (e != hipSuccess) return e;
-  hipLaunchKernelGGL(fn, dim3(grid), dim3(64 * WAVES), lds, st, a, causal);
+  // (short-context units: kv heads along x, so that a record's run together)
+  const dim3 g = KIND == DecodeKind::Short ? dim3(a.hkv, grid / a.hkv) : dim3(grid);
+  hipLaunchKernelGGL(fn, g, dim3(64 * WAVES), lds, st, a, causal);
   return hipGetLastError();
 }
 

@@ -25,7 +25,10 @@ typedef int32_t i32x8 __attribute__((ext_vector_type(8)));
 // memory round trip after its record (the record names the first 64 tokens'
 // blocks of every wavefront).  Then S^T, one softmax step and O^T += V^T P^T
 // over the 64 tokens as in the tile kernel.
-template <bool BF16, int WAVES, int NCB>
+// GRID2: a workgroup's unit is (record blockIdx.y, kv head blockIdx.x); else
+// the workgroups loop over n_items units (a graph's grid covers any prepare's),
+// at the price of a division (0.05 us).
+template <bool BF16, int WAVES, int NCB, bool GRID2>
 __device__ __forceinline__ void short_items(const AttnArgs& a, int causal, int n_items, uint8_t* dsm) {
   const int lane = threadIdx.x & 63;
   const int J = lane >> 4;
@@ -56,13 +59,15 @@ __device__ __forceinline__ void short_items(const AttnArgs& a, int causal, int n
     }
   }
 
-  for (int it = blockIdx.x; it < n_items; it += gridDim.x) {
-    const ShortItem* rec = a.shorts + uniform(it);
+  for (int it = GRID2 ? 0 : blockIdx.x; it < n_items; it += gridDim.x) {
+    const int ri = GRID2 ? (int)blockIdx.y : uniform(it / a.hkv);
+    const int kvh = GRID2 ? (int)blockIdx.x : uniform(it) - ri * a.hkv;
+    const ShortItem* rec = a.shorts + ri;
     typedef const __attribute__((address_space(4))) i32x8* c_i32x8;
     typedef const __attribute__((address_space(4))) i32x4* c_i32x4;
     const i32x8 h = *(c_i32x8)rec;
     const i32x4 first = *(c_i32x4)(rec->block + 4 * wave);
-    const int q0 = h[0], nq = h[1], kvh = h[2], vis = h[3], t0 = h[4], t1 = h[5], part = h[6], page_off = h[7];
+    const int q0 = h[0], nq = h[1], vis = h[2], t0 = h[3], t1 = h[4], part = h[5], page_off = h[6];
     const int ncols = nq * G;
     const int nblk = (t1 - t0 + 15) >> 4;
     const int nbw = (nblk + WAVES - 1) / WAVES;     // blocks per wavefront
@@ -285,6 +290,7 @@ __device__ __forceinline__ void short_items(const AttnArgs& a, int causal, int n
         if (c == 0) a.part_lse[oi] = l2;
       }
     }
+    if constexpr (GRID2) break;
     if (it + (int)gridDim.x < n_items) __syncthreads();  // the regions are the next item's V
   }
 }

@@ -69,15 +69,17 @@ struct alignas(64) ShareStart {
   int32_t pg0;
   int32_t pg1;
   int32_t n_short;  // in every record, so that a graph launch need not read the header first: > 0 when the
-                    // batch is planned as that many ShortItem records at the heap's start and no shares
+                    // batch is planned as that many short-context units (ShortItem records at the heap's
+                    // start, hkv units each) and no shares
   int32_t pad[3];
 };
 static_assert(sizeof(ShareStart) == 64, "one 64-byte scalar load");
 static_assert(sizeof(DecodeItem) == 32, "two pieces per 64 bytes");
 
-// One workgroup's unit of the short-context kernel: query rows [q0, q0+nq)
-// (all the query heads of kv head `kvh`, at most kDecodeCols columns) against
-// tokens [t0, t1), t0 a multiple of 16; part as in WorkItem.  Its 16-token
+// hkv units (workgroups) of the short-context kernel, one per kv head: query
+// rows [q0, q0+nq) (all the query heads of the kv head, at most kDecodeCols
+// columns) against tokens [t0, t1), t0 a multiple of 16; part as in WorkItem.
+// Unit i is record i / hkv, kv head i % hkv.  A unit's 16-token
 // blocks are divided evenly among the workgroup's W wavefronts (wavefront w:
 // blocks [w * n, (w + 1) * n) of the item, n = ceil(blocks / W)); `block`
 // names the first four of every wavefront by their index in the cache in
@@ -86,12 +88,12 @@ static_assert(sizeof(DecodeItem) == 32, "two pieces per 64 bytes");
 struct alignas(32) ShortItem {
   int32_t q0;
   int32_t nq;
-  int32_t kvh;
   int32_t vis;       // last token that row q0 sees under the causal mask
   int32_t t0;
   int32_t t1;
   int32_t part;
   int32_t page_off;  // index of the sequence's first page id
+  int32_t pad;
   int32_t block[4 * kDecodeWavesPerCu];
 };
 static_assert(sizeof(ShortItem) == 160, "record and block list in two scalar loads");
@@ -121,7 +123,7 @@ struct AttnArgs {
   const ShareStart* shares;  // decode only: one record per share
   int n_share_cap;           // decode only: records in `shares`
   const ShortItem* shorts;   // short-context kernel: the items (graph launches: the heap's start)
-  int n_short;               // short-context kernel, eager launches: items at `shorts`
+  int n_short;               // short-context kernel, eager launches: units (hkv per record)
   uint16_t* part_o;        // [slots][hq][128] in the attention's 16-bit type, normalised per split
   float* part_lse;         // [slots][hq] log2 domain
   int hq;

@@ -269,7 +269,7 @@ int write_image(uint8_t* h, const Layout& l, const HeapPlace& hp, const PlanShap
   std::memset(ss + n_shares, 0, sizeof(ShareStart) * (size_t)(scap - n_shares));
   const std::vector<ShortItem>& shorts = bp.shorts;
   if (!shorts.empty())
-    for (int k = 0; k < scap; ++k) ss[k].n_short = (int32_t)shorts.size();
+    for (int k = 0; k < scap; ++k) ss[k].n_short = (int32_t)shorts.size() * sh.hkv;
   ShortItem* sp = reinterpret_cast<ShortItem*>(heap + hp.shorts);
   for (size_t i = 0; i < shorts.size(); ++i) {
     sp[i] = shorts[i];
@@ -319,7 +319,7 @@ struct Launch {
   bool wide_merge[2] = {false, false};
   int64_t rows = 0;  // query rows of the sequences
   size_t merge_off[2] = {0, 0};  // heap offsets of the merge lists just staged
-  int n_short = 0;
+  int n_short = 0;  // short-context units
   int n_tshare[2] = {0, 0};  // tile shares (workgroups) in use per mask mode
   int decode_wg = 8;         // wavefronts per decode workgroup
   int decode_nc = 16;
@@ -360,7 +360,7 @@ void record_lists(Launch& L, const BuiltPlan& bp, const HeapPlace& hp, int nc) {
   for (const SeqInfo& s : bp.seqs) L.rows += s.qlen;
   L.decode_nc = nc;
   for (int m = 0; m < 2; ++m) L.merge_off[m] = hp.merge[m];
-  L.n_short = (int)bp.shorts.size();
+  L.n_short = (int)bp.shorts.size() * L.sh.hkv;
   L.n_decode = (int)bp.decode_starts.size() * L.sh.hkv;  // busy decode wavefronts
   for (int m = 0; m < 2; ++m) {
     L.n_tile[m] = (int)bp.mode[m].tile.size();

@@ -57,6 +57,12 @@ void assign_shares(std::vector<WorkItem>& items, int slots, std::vector<int32_t>
                      [](const WorkItem& x, const WorkItem& y) { return x.cost > y.cost; });
   }
   const int n = std::max(1, std::min<int>(slots, (int)items.size()));
+  if (!items.empty() && (int)items.size() <= slots && items.back().cost > 0) {
+    // A share for every item: each goes to the first that is still empty.
+    off.resize((size_t)n + 1);
+    for (int k = 0; k <= n; ++k) off[k] = k;
+    return;
+  }
   std::vector<int> share(items.size());
   // Binary min-heap of (load << 20 | share) keys: the root is the least-loaded
   // share, the lowest index among equals.  Each item raises the root's load
@@ -244,14 +250,21 @@ bool plan_short(const PlanShape& sh, const int32_t* pages, int waves, BuiltPlan&
   std::vector<int> order;
   for (int b = 0; b < (int)out.seqs.size(); ++b)
     if (out.seqs[b].qlen > 0) order.push_back(b);
-  std::stable_sort(order.begin(), order.end(), [&](int x, int y) { return out.seqs[x].len > out.seqs[y].len; });
+  auto longer = [&](int x, int y) { return out.seqs[x].len > out.seqs[y].len; };
+  if (!std::is_sorted(order.begin(), order.end(), longer)) std::stable_sort(order.begin(), order.end(), longer);
+  int in_page = 0;  // log2 of the 16-token blocks of a page
+  while ((16 << in_page) < sh.page) ++in_page;
+  const int block_mask = (1 << in_page) - 1;
   ModeLists ml;
   std::vector<ShortItem> items;
-  items.reserve((size_t)(max_len <= piece ? whole : cut));
+  items.reserve((size_t)((max_len <= piece ? whole : cut) / sh.hkv));
   for (int b : order) {
     const SeqInfo& s = out.seqs[b];
-    const int len = round_up(ceil_div(s.len, ceil_div(s.len, piece)), 16);  // of one piece
-    const int np = ceil_div(s.len, len);
+    int len = s.len, np = 1;  // of one piece; pieces
+    if (s.len > piece) {
+      len = round_up(ceil_div(s.len, ceil_div(s.len, piece)), 16);
+      np = ceil_div(s.len, len);
+    }
     int base = -1;
     if (np > 1) {
       base = ml.partial_rows;
@@ -259,7 +272,8 @@ bool plan_short(const PlanShape& sh, const int32_t* pages, int waves, BuiltPlan&
       for (int r = 0; r < s.qlen; ++r) ml.merge.push_back(MergeRow{s.qo + r, base + r, np, s.qlen});
     }
     for (int p = 0; p < np; ++p) {
-      ShortItem it{};
+      items.emplace_back();  // for every kv head
+      ShortItem& it = items.back();
       it.q0 = s.qo;
       it.nq = s.qlen;
       it.vis = s.len - s.qlen;
@@ -269,18 +283,13 @@ bool plan_short(const PlanShape& sh, const int32_t* pages, int waves, BuiltPlan&
       it.page_off = s.page_off;
       const int nblk = ceil_div(it.t1 - it.t0, 16);
       const int per = ceil_div(nblk, waves);
-      for (int w = 0; w * per < nblk; ++w) {
-        const int end = std::min(nblk, (w + 1) * per);
+      const int32_t* pg = pages + s.page_off;
+      int32_t* dst = it.block;
+      for (int b0 = it.t0 >> 4, end = b0 + nblk; b0 < end; b0 += per)  // a wavefront's blocks
         for (int j = 0; j < 4; ++j) {
-          const int tok = it.t0 + 16 * std::min(w * per + j, end - 1);
-          it.block[4 * w + j] = (int32_t)((uint32_t)pages[s.page_off + tok / sh.page] * (uint32_t)(sh.page / 16) +
-                                          (uint32_t)(tok % sh.page / 16));
+          const int blk = std::min(b0 + j, std::min(end, b0 + per) - 1);
+          *dst++ = (int32_t)(((uint32_t)pg[blk >> in_page] << in_page) + (uint32_t)(blk & block_mask));
         }
-      }
-      for (int h = 0; h < sh.hkv; ++h) {
-        it.kvh = h;
-        items.push_back(it);
-      }
     }
   }
   if (ml.partial_rows > sh.partial_cap || ml.merge.size() > (size_t)sh.partial_cap) return false;

@@ -42,7 +42,8 @@ struct BuiltPlan {
   std::vector<ShareStart> decode_starts;  // one per share in use
   int decode_partials = 0;
   std::vector<MergeRow> decode_merge;
-  std::vector<ShortItem> shorts;  // the whole batch as short-context items (then no other items); both masks
+  std::vector<ShortItem> shorts;  // the whole batch as short-context items (then no other items), one record for
+                                  // all kv heads; both masks
   int decode_nc = 16;            // 16 or 32 columns per decode item (MFMA column blocks x 16)
   ModeLists mode[2];             // [0] full (non-causal), [1] causal
 };

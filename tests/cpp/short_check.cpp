@@ -1,7 +1,7 @@
 // Short-context plans (planner.hpp: build_plan with short_waves > 0) over
 // random batches: where the planner takes that form, its items cover every
-// (query row, kv head, visible token) once with both masks, their block
-// lists name the pages the page table does, split rows have partial slots of
+// (query row, visible token) once with both masks, their block lists
+// name the pages the page table does, split rows have partial slots of
 // their own inside the budget and a merge record each, and no other list is
 // filled.  Where it does not, the plan is the ordinary one.  Host code only;
 // built and run by tests/test_short_plan.py.
@@ -90,18 +90,18 @@ static bool check(const Case& c, int waves, int& taken) {
     CHECK(ml.tile.empty() && ml.tile_off.empty());
     CHECK((int64_t)bp.shorts.size() * (int64_t)sizeof(ShortItem) <= (int64_t)c.sh.item_cap * (int64_t)sizeof(WorkItem));
     CHECK(ml.partial_rows <= c.sh.partial_cap && (int)ml.merge.size() <= c.sh.partial_cap);
-    // (row, kv head) -> pieces; partial slot -> owners
-    std::map<std::pair<int, int>, std::vector<const ShortItem*>> cover;
+    // row -> pieces (a record stands for every kv head); partial slot -> owners
+    std::map<int, std::vector<const ShortItem*>> cover;
     std::map<int, std::set<int>> slot_rows;
     for (const ShortItem& w : bp.shorts) {
-      CHECK(w.nq >= 1 && w.nq * G <= bp.decode_nc && w.kvh >= 0 && w.kvh < c.sh.hkv);
+      CHECK(w.nq >= 1 && w.nq * G <= bp.decode_nc);
       CHECK(w.t0 >= 0 && w.t0 % 16 == 0 && w.t1 > w.t0);
       const int b = (int)(std::upper_bound(c.qo.begin(), c.qo.end(), w.q0) - c.qo.begin()) - 1;
       const SeqInfo& s = bp.seqs[b];
       CHECK(w.q0 >= s.qo && w.q0 + w.nq <= s.qo + s.qlen && w.page_off == s.page_off && w.t1 <= s.len);
       CHECK(w.vis == s.len - s.qlen + (w.q0 - s.qo));
       for (int r = 0; r < w.nq; ++r) {
-        cover[{w.q0 + r, w.kvh}].push_back(&w);
+        cover[w.q0 + r].push_back(&w);
         if (w.part >= 0) {
           CHECK(w.part + r < ml.partial_rows);
           slot_rows[w.part + r].insert(w.q0 + r);
@@ -126,24 +126,22 @@ static bool check(const Case& c, int waves, int& taken) {
       for (int i = 0; i < bp.seqs[b].qlen; ++i) {
         const SeqInfo& s = bp.seqs[b];
         const int row = s.qo + i, seen = causal ? s.len - s.qlen + i + 1 : s.len;
-        for (int h = 0; h < c.sh.hkv; ++h) {
-          ++rows;
-          std::vector<const ShortItem*>& v = cover[{row, h}];
-          std::sort(v.begin(), v.end(), [](const ShortItem* x, const ShortItem* y) { return x->t0 < y->t0; });
-          int at = 0;
-          for (size_t p = 0; p < v.size(); ++p) {
-            CHECK(v[p]->t0 == at);
-            at = v[p]->t1;
-            if (v.size() > 1) {
-              CHECK(merge.count(row) == 1);
-              const MergeRow& m = merge[row];
-              CHECK(m.nsplit == (int)v.size() && v[p]->part + (row - v[p]->q0) == m.part + (int)p * m.stride);
-            } else {
-              CHECK(v[p]->part == -1 && merge.count(row) == 0);
-            }
+        ++rows;
+        std::vector<const ShortItem*>& v = cover[row];
+        std::sort(v.begin(), v.end(), [](const ShortItem* x, const ShortItem* y) { return x->t0 < y->t0; });
+        int at = 0;
+        for (size_t p = 0; p < v.size(); ++p) {
+          CHECK(v[p]->t0 == at);
+          at = v[p]->t1;
+          if (v.size() > 1) {
+            CHECK(merge.count(row) == 1);
+            const MergeRow& m = merge[row];
+            CHECK(m.nsplit == (int)v.size() && v[p]->part + (row - v[p]->q0) == m.part + (int)p * m.stride);
+          } else {
+            CHECK(v[p]->part == -1 && merge.count(row) == 0);
           }
-          CHECK(at >= seen && at <= s.len);
         }
+        CHECK(at >= seen && at <= s.len);
       }
     CHECK(rows == cover.size());
   }
