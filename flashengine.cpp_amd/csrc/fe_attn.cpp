@@ -316,6 +316,7 @@ struct Launch {
   bool tile_stream[2] = {true, true};  // tile K/V reads with the non-temporal hint, per mask mode
   int graph_stream[2] = {-1, -1};      // graph plans: that choice at the first graph prepare
   int n_decode = 0, n_tile[2] = {0, 0}, n_merge[2] = {0, 0};
+  int n_pieces = 0, tile_rows[2] = {0, 0};  // reported only
   bool wide_merge[2] = {false, false};
   int64_t rows = 0;  // query rows of the sequences
   size_t merge_off[2] = {0, 0};  // heap offsets of the merge lists just staged
@@ -362,8 +363,10 @@ void record_lists(Launch& L, const BuiltPlan& bp, const HeapPlace& hp, int nc) {
   for (int m = 0; m < 2; ++m) L.merge_off[m] = hp.merge[m];
   L.n_short = (int)bp.shorts.size() * L.sh.hkv;
   L.n_decode = (int)bp.decode_starts.size() * L.sh.hkv;  // busy decode wavefronts
+  L.n_pieces = (int)bp.decode_items.size() * L.sh.hkv;
   for (int m = 0; m < 2; ++m) {
     L.n_tile[m] = (int)bp.mode[m].tile.size();
+    L.tile_rows[m] = bp.mode[m].tile.empty() ? 0 : bp.mode[m].tile_rows;
     L.n_tshare[m] = bp.mode[m].tile_off.empty() ? 0 : (int)bp.mode[m].tile_off.size() - 1;
     L.n_merge[m] = (int)bp.mode[m].merge.size();
     L.wide_merge[m] = merge_wide(bp.mode[m].merge, L.sh);
@@ -726,6 +729,17 @@ int fe_attn_run(fe_attn_plan* p, const void* q, const void* k_cache, const void*
   rc = check_stream_device(static_cast<hipStream_t>(stream), p->device);
   if (rc != FE_OK) return rc;
   return launch_all(p->run, q, k_cache, v_cache, out, lse, causal, static_cast<hipStream_t>(stream));
+}
+
+int fe_attn_plan_lists(const fe_attn_plan* p, int causal, int32_t* counts_out) {
+  if (p == nullptr || counts_out == nullptr) return fail(FE_EINVAL, "plan lists: null pointer");
+  if (!p->prepared) return fail(FE_EINVAL, "plan lists called before prepare_plan");
+  const Launch& L = p->run;
+  const int m = causal ? 1 : 0;
+  const int32_t counts[] = {L.n_pieces,   L.n_short,  L.n_tile[m], L.tile_rows[m],
+                            L.n_merge[m], L.wide_merge[m] ? 1 : 0, L.tile_stream[m] ? 1 : 0};
+  std::memcpy(counts_out, counts, sizeof(counts));
+  return FE_OK;
 }
 
 int fe_rope_table(float* table, int max_len, int dim, double theta, void* stream) {

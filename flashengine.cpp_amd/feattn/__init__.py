@@ -15,7 +15,7 @@ from __future__ import annotations
 
 import ctypes
 import os
-from typing import Optional, Sequence
+from typing import NamedTuple, Optional, Sequence
 
 PKG_DIR = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
 LIB_PATH = os.environ.get("FEATTN_LIB") or os.path.join(PKG_DIR, "lib", "libfeattn.so")
@@ -36,6 +36,7 @@ C_SYMBOLS = (
     "fe_store",
     "fe_rope_append",
     "fe_attn_last_error",
+    "fe_attn_plan_lists",
     "fe_attn_plan_describe",
     "fe_attn_plan_dump",
     "fe_attn_version",
@@ -110,6 +111,7 @@ def lib() -> ctypes.CDLL:
     L.fe_rope.argtypes = [_vp, _vp, _vp, _vp, _int, _int, _int, _int, _int, _vp, _int]
     L.fe_store.argtypes = [_vp, _vp, _vp, _vp, _vp, _int, _int, _int, _vp, _int]
     L.fe_rope_append.argtypes = [_vp] * 8 + [_int] * 7 + [_vp]
+    L.fe_attn_plan_lists.argtypes = [_vp, _int, _i32p]
     L.fe_attn_plan_describe.argtypes = [_int] * 7 + [_i32p] * 4 + [_int, _int, _i32p]
     L.fe_attn_plan_dump.argtypes = [_int] * 7 + [_i32p] * 4 + [_int, _int, _int, _i32p, _int,
                                                              ctypes.POINTER(_int)]
@@ -176,6 +178,17 @@ def _ptr(t) -> Optional[int]:
     return None if t is None else t.data_ptr()
 
 
+class PlanLists(NamedTuple):
+    """Counts of a prepared plan's work lists (fe_attn_plan_lists)."""
+    decode_items: int
+    short_units: int
+    tile_items: int
+    tile_rows: int
+    merge_rows: int
+    merge_wide: int
+    tile_stream: int
+
+
 class Plan:
     """Owning wrapper of ``fe_attn_plan`` (reference: fe::cuda::AttentionPlan,
     created with create_plan's arguments, native_cuda.hpp:7)."""
@@ -202,6 +215,12 @@ class Plan:
         """fe::cuda::attention (native_cuda.hpp:10) plus the optional LSE output."""
         _check(lib().fe_attn_run(self._h, _ptr(q), _ptr(k_cache), _ptr(v_cache), _ptr(out),
                                  _ptr(lse), int(bool(causal)), _stream(stream)))
+
+    def lists(self, causal: bool = True) -> PlanLists:
+        """What the latest prepare planned for run(causal=causal) (fe_attn_plan_lists)."""
+        out = (ctypes.c_int32 * 7)()
+        _check(lib().fe_attn_plan_lists(self._h, int(bool(causal)), out))
+        return PlanLists(*out)
 
     def close(self) -> None:
         if getattr(self, "_h", None) is not None and self._h.value:
@@ -249,7 +268,7 @@ def rope_append(q, k, v, k_cache, v_cache, pos, slots, cache, rows: int, hq: int
 
 
 def describe(hq, hkv, dim, page, max_batch, max_pages, blocks, qo, kv, pages, last, batch, rows):
-    """Host-only planner counts: (decode items, causal tile items, merge rows, partial rows)."""
+    """Host-only counts of the general plan: (decode items, causal tile items, merge rows, partial rows)."""
     out = (ctypes.c_int32 * 4)()
     _check(lib().fe_attn_plan_describe(hq, hkv, dim, page, max_batch, max_pages, blocks, _i32(qo),
                                        _i32(kv), _i32(pages), _i32(last), batch, rows, out))
@@ -270,7 +289,7 @@ def assign_shares(costs: Sequence[int], slots: int, fast: int = -1):
 
 def dump(hq, hkv, dim, page, max_batch, max_pages, blocks, qo, kv, pages, last, batch, rows,
          causal: bool):
-    """Host-only planner work list: list of (kind, seq, q0, nq, kvh, t0, t1, part)."""
+    """Host-only work list of the general plan: list of (kind, seq, q0, nq, kvh, t0, t1, part)."""
     n = _int()
     _check(lib().fe_attn_plan_dump(hq, hkv, dim, page, max_batch, max_pages, blocks, _i32(qo),
                                    _i32(kv), _i32(pages), _i32(last), batch, rows, int(causal),

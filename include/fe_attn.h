@@ -155,19 +155,28 @@ int fe_attn_run_noalloc(const void* q, const void* k_cache, const void* v_cache,
 /* Message of the last failed call on this thread ("" if none). */
 const char* fe_attn_last_error(void);
 
+/* The work lists of the plan's latest prepare, as fe_attn_run with this
+ * `causal` launches them.  counts_out[0..6] = decode items, short-context
+ * units (then no decode items), tile items, query rows of a tile item at
+ * most, merge rows, form of the merge (0 a wavefront, 1 a workgroup per row
+ * and pair of heads), tile reads with the non-temporal hint (0/1).  For
+ * callers and tests that want to know which form a batch was given. */
+int fe_attn_plan_lists(const fe_attn_plan* plan, int causal,
+                       int32_t* counts_out);
+
 /* Host-only planner introspection (no device needed): runs the same
  * validation as fe_attn_plan_prepare and reports the counts of the general
- * plan (shares and full-width tile items; prepare plans small calls in other
- * forms where those are faster).  Used by tests and by the benchmark to report the split-KV
- * layout.  counts_out[0..3] = decode items, tile items, merge rows,
- * partial rows. */
+ * plan (shares and full-width tile items).  prepare plans small calls in
+ * other forms where those are faster: fe_attn_plan_lists reports what it
+ * chose.  counts_out[0..3] = decode items, tile items, merge rows, partial
+ * rows. */
 int fe_attn_plan_describe(int hq, int hkv, int dim, int page, int max_batch,
                           int max_pages, int blocks, const int32_t* qo,
                           const int32_t* kv, const int32_t* pages,
                           const int32_t* last, int batch, int rows,
                           int32_t* counts_out);
 
-/* Host-only planner dump: writes up to `cap` work items (8 int32 each:
+/* Host-only planner dump of the same general plan: writes up to `cap` work items (8 int32 each:
  * kind(0 decode,1 tile), seq, q0, nq, kvh, t0, t1, part) and returns the
  * number written in *n_out.  Lets CPU tests check that every visible
  * (row, head, token) triple is covered exactly once. */

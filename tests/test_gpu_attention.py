@@ -140,9 +140,10 @@ def test_causal_prefix_known_answer(dev):
 def test_split_kv_long_context(dev):
     b = W.long_decode(batch=3, ctx=32768)
     q, kc, vc = W.make_tensors(b, seed=6)
-    counts = feattn.describe(b.hq, b.hkv, 128, 16, b.batch, b.max_pages(), b.blocks, b.qo, b.kv,
-                             b.pages, b.last, b.batch, b.rows)
-    assert counts[2] == 3  # split + merged
+    plan = feattn.Plan(b.hq, b.hkv, 128, 16, b.batch, b.max_pages(), True, b.blocks)
+    plan.prepare(b.qo, b.kv, b.pages, b.last, b.batch, b.rows)
+    assert plan.lists().merge_rows == 3  # split + merged
+    plan.close()
     out, lse = hip_attention(b, q, kc, vc, True, dev)
     want_out, want_lse = A.run(b, q, kc, vc, True)
     check(out, lse, want_out, want_lse)
@@ -221,9 +222,11 @@ def test_shared_prefix_pages_vs_oracle(dev, causal, dtype):
     """Decode, block, chunk and split-KV work over page tables that share
     pages across sequences, against the oracle."""
     b = shared_prefix_batch()
-    counts = feattn.describe(b.hq, b.hkv, 128, 16, b.batch, b.max_pages(), b.blocks, b.qo, b.kv,
-                             b.pages, b.last, b.batch, b.rows)
-    assert counts[0] > 0 and counts[1] > 0 and counts[2] > 0  # decode, tile and merged (split) rows
+    plan = feattn.Plan(b.hq, b.hkv, 128, 16, b.batch, b.max_pages(), dtype == "bf16", b.blocks)
+    plan.prepare(b.qo, b.kv, b.pages, b.last, b.batch, b.rows)
+    got = plan.lists(causal)
+    plan.close()
+    assert got.decode_items > 0 and got.tile_items > 0 and got.merge_rows > 0  # merged: split rows
     q, kc, vc = W.make_tensors(b, seed=78, dtype=dtype)
     want_out, want_lse = A.run(b, q, kc, vc, causal)
     out, lse = hip_attention(b, q, kc, vc, causal, dev)

@@ -165,9 +165,10 @@ def test_counts_single_128k_sequence(dev):
     the 1e-5 bound, so this pins the count to within a token (and any lost
     or doubled piece by far)."""
     b = W.make_batch(32, 8, starts=[131071, 5], qlens=[1, 1], seed=128, extra_pages=1)
-    counts = feattn.describe(b.hq, b.hkv, 128, b.page, b.batch, b.max_pages(), b.blocks, b.qo, b.kv,
-                             b.pages, b.last, b.batch, b.rows)
-    assert counts[3] >= 128  # the long row is cut into that many partial rows at least
+    plan = feattn.Plan(b.hq, b.hkv, 128, b.page, b.batch, b.max_pages(), False, b.blocks)
+    plan.prepare(b.qo, b.kv, b.pages, b.last, b.batch, b.rows)
+    assert plan.lists().decode_items >= 128 * 8  # the long row is cut into that many pieces at least
+    plan.close()
     run_case(dev, b, True, "f16")
 
 
@@ -218,4 +219,10 @@ def test_exact_counts_tile_stream_cut(dev, name, causal):
     hq, hkv, starts, qlens = STREAM_CUT[name]
     b = W.make_batch(hq, hkv, starts=starts, qlens=qlens, seed=hq + hkv + 5, extra_pages=1)
     assert stream_cut_taken(b, causal)
+    items = [it for it in feattn.dump(hq, hkv, 128, b.page, b.batch, b.max_pages(), b.blocks, b.qo, b.kv, b.pages,
+                                      b.last, b.batch, b.rows, causal) if it[0] == 1]
+    plan = feattn.Plan(hq, hkv, 128, b.page, b.batch, b.max_pages(), False, b.blocks)
+    plan.prepare(b.qo, b.kv, b.pages, b.last, b.batch, b.rows)
+    assert plan.lists(causal).tile_items == len(items)  # prepare takes that list
+    plan.close()
     run_case(dev, b, causal, "f16")

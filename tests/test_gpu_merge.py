@@ -23,15 +23,15 @@ def test_split_counts(dev, dtype, rows):
     graph_plan = feattn.Plan(hq, hkv, 128, 16, 2, 600, dtype == "bf16", 1200)
     for lens in ([64 * 130 + 7], [64 * 8], [64 * 8 + 1], [64 * 16 + 1], [64 * 64], [64 * 64 + 1], [70, 64 * 17]):
         b = W.make_batch(hq, hkv, starts=[n - rows for n in lens], qlens=[rows] * len(lens), seed=lens[0], pool=1200)
-        counts = feattn.describe(hq, hkv, 128, 16, 2, 600, 1200, b.qo, b.kv, b.pages, b.last, b.batch, b.rows)
-        if len(lens) == 1:
-            assert counts[3] == -(-lens[0] // 64) * rows  # partial rows
         q, kc, vc = W.make_tensors(b, seed=3, dtype=dtype)
         want, want_lse = A.run(b, q, kc, vc, True)
         q, kc, vc = q.to(dev), kc.to(dev), vc.to(dev)
         got = []
         for p, graph in ((plan, False), (graph_plan, True)):
             p.prepare(b.qo, b.kv, b.pages, b.last, b.batch, b.rows, graph=graph)
+            forms = p.lists()
+            assert forms.decode_items == sum(-(-n // 64) for n in lens) * hkv or len(lens) > 1
+            assert forms.merge_rows == rows * len(lens) and forms.merge_wide == int(max(lens) > 8 * 64)
             out = torch.full_like(q, float("nan"))
             lse = torch.full((b.rows, hq), float("nan"), device=dev)
             p.run(q, kc, vc, out, causal=True, lse=lse)

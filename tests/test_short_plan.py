@@ -72,6 +72,7 @@ def test_short_kernel_edges(dev, hq, hkv, rows, page, dtype, causal):
 
         plan.prepare(b.qo, b.kv, b.pages, b.last, b.batch, b.rows)
         graph_plan.prepare(b.qo, b.kv, b.pages, b.last, b.batch, b.rows, graph=True)
+        assert plan.lists(causal).short_units > 0 and graph_plan.lists(causal).short_units > 0
         got = [run(plan), run(graph_plan)]
         if graph is None:
             sq, sk, sv = qd.clone(), kd.clone(), vd.clone()
@@ -92,6 +93,73 @@ def test_short_kernel_edges(dev, hq, hkv, rows, page, dtype, causal):
             assert torch.equal(out, got[0][0]) and torch.equal(lse, got[0][1])
     plan.close()
     graph_plan.close()
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("hq,hkv,rows,page", [(32, 8, 1, 16), (16, 8, 1, 64), (40, 8, 5, 16), (8, 8, 8, 32),
+                                              (32, 8, 8, 16), (32, 4, 1, 16), (32, 4, 4, 32), (64, 4, 1, 16)])
+@pytest.mark.parametrize("dtype,causal", [("bf16", True), ("f16", False)])
+def test_share_kernel_edges(dev, hq, hkv, rows, page, dtype, causal):
+    """The same lengths beside a chunk, which puts them on the decode shares
+    (as long contexts are): the same edges of that kernel, eagerly and
+    through a graph plan, which must give the same bits."""
+    lens = [max(n, rows) for n in LENS[hkv]] + [70]
+    b = W.make_batch(hq, hkv, starts=[n - rows for n in lens[:-1]] + [0], qlens=[rows] * (len(lens) - 1) + [70],
+                     seed=len(lens), page=page, extra_pages=2)
+    q, kc, vc = W.make_tensors(b, seed=8, dtype=dtype)
+    want, want_lse = A.run(b, q, kc, vc, causal)
+    used = torch.zeros((b.blocks + 1) * page, dtype=torch.bool)
+    for s in range(b.batch):
+        for t in range(b.lens[s]):
+            used[b.tables[s][t // page] * page + t % page] = True
+    used = used.view(b.blocks + 1, page)
+    kc[~used] = float("nan")
+    vc[~used] = float("nan")
+    q, kc, vc = q.to(dev), kc.to(dev), vc.to(dev)
+    got = []
+    for graph in (False, True):
+        plan = feattn.Plan(hq, hkv, 128, page, b.batch, b.max_pages(), dtype == "bf16", b.blocks)
+        plan.prepare(b.qo, b.kv, b.pages, b.last, b.batch, b.rows, graph=graph)
+        forms = plan.lists(causal)
+        assert forms.short_units == 0 and forms.decode_items > 0 and forms.merge_rows > 0
+        out = torch.full_like(q, float("nan"))
+        lse = torch.full((b.rows, hq), float("nan"), device=dev)
+        plan.run(q, kc, vc, out, causal=causal, lse=lse)
+        torch.cuda.synchronize()
+        plan.close()
+        torch.testing.assert_close(out.float().cpu(), want.float(), atol=1e-2, rtol=1e-2)
+        torch.testing.assert_close(lse.cpu(), want_lse, atol=1e-3, rtol=0)
+        got.append((out, lse))
+    assert torch.equal(got[0][0], got[1][0]) and torch.equal(got[0][1], got[1][1])
+
+
+# (heads, cached tokens, new tokens, masks): the lists a plan reports, eagerly
+# and for a graph.
+FORMS = [
+    (32, 8, [63] * 4, [1] * 4, dict(short_units=4 * 8, decode_items=0, merge_rows=0)),
+    (32, 8, [700, 30], [1, 1], dict(short_units=3 * 8, merge_rows=1)),
+    (32, 8, [3000] * 12, [1] * 12, dict(short_units=0, merge_rows=12, tile_items=0)),
+    (5, 5, [300], [1], dict(short_units=0, decode_items=25, merge_rows=1, merge_wide=0)),
+    (5, 5, [700], [1], dict(short_units=0, decode_items=55, merge_rows=1, merge_wide=1)),
+    (16, 8, [0], [100], dict(short_units=0, tile_items=32, tile_rows=32, merge_rows=0)),
+    (16, 8, [4000], [100], dict(tile_rows=64, merge_rows=100)),
+    (32, 8, [60, 0], [1, 100], dict(short_units=0, tile_items=56, tile_rows=16)),
+]
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("hq,hkv,starts,qlens,want", FORMS)
+@pytest.mark.parametrize("graph", [False, True])
+def test_lists_report_the_prepared_form(dev, hq, hkv, starts, qlens, want, graph):
+    b = W.make_batch(hq, hkv, starts=starts, qlens=qlens, seed=1)
+    plan = feattn.Plan(hq, hkv, 128, 16, b.batch, b.max_pages(), True, b.blocks)
+    with pytest.raises(RuntimeError, match="before prepare"):
+        plan.lists()
+    plan.prepare(b.qo, b.kv, b.pages, b.last, b.batch, b.rows, graph=graph)
+    for causal in (True, False):
+        got = plan.lists(causal)._asdict()
+        assert {k: got[k] for k in want} == want
+    plan.close()
 
 
 @pytest.mark.gpu
