@@ -5,9 +5,9 @@
 // time from the capacity arguments, like the reference's FlashInfer plan
 // (src/flashinfer_attention.cu:14-27).  prepare() builds the work lists on
 // the host into a pinned mirror of the arena and stages them with one copy
-// on the caller's stream; run() only launches kernels, whose grids depend on
-// the plan capacity in graph mode, so a captured graph stays valid across
-// prepares.
+// on the caller's stream; run() only launches kernels, whose grids in graph
+// mode cover the plan capacity or loop over what exceeds them, so a captured
+// graph stays valid across prepares.
 #include "fe_attn.h"
 #include "fe_driver.h"
 #include "fe_ops.h"
@@ -333,7 +333,7 @@ void init_launch(Launch& L, const PlanShape& sh, bool bf16) {
   L.decode_wg = decode_wg_waves(sh.hkv);
   L.grid_decode_cap = sh.num_cus * kDecodeWavesPerCu / L.decode_wg;  // persistent: every workgroup resident
   L.grid_tile_cap = sh.tile_slots;
-  L.grid_merge_cap = sh.num_cus * 8;  // 4 (row, head pair) units per workgroup
+  L.grid_merge_cap = sh.num_cus * 8;
 }
 
 // Launch sizes of the lists just staged.
@@ -376,6 +376,27 @@ void record_lists(Launch& L, const BuiltPlan& bp, const HeapPlace& hp, int nc) {
     if (L.graph && L.graph_stream[m] < 0) L.graph_stream[m] = once ? 1 : 0;
     L.tile_stream[m] = L.graph ? L.graph_stream[m] > 0 : once;
   }
+}
+
+// Workgroups of the merge launch: one per row and pair of heads (wide form) or
+// per four of them.  A decode graph's launch has a workgroup for every row and
+// pair of the latest prepare, of max_batch single rows, and for every four of
+// max_batch sequences of as many rows as the captured decode variant takes, so
+// that whatever the batch it was captured on, a later one of the plan's size
+// is folded in one pass: captured on 1 sequence of a plan for 64 and replayed
+// on 64 x 3000 tokens 118.6 us, with a grid for the 1 row 129.7; 12 x 2000 of a
+// plan for 12, 21.9 and 39.0.  (As many as the launch cap, mostly idle, take 0.5
+// us a call more on 12 sequences.)  Beside a tile kernel the rows of a later
+// batch have no such bound: there the cap.
+int merge_grid(const Launch& L, int mode) {
+  const int64_t hpairs = (L.sh.hq + 1) / 2;
+  int64_t wgs = L.wide_merge[mode] ? L.n_merge[mode] * hpairs : (L.n_merge[mode] * hpairs + 3) / 4;
+  if (L.graph) {
+    const int64_t seq_rows = std::max(1, L.decode_nc / (L.sh.hq / L.sh.hkv));
+    wgs = L.graph_tile > 0 ? L.grid_merge_cap
+                           : hpairs * std::max<int64_t>({L.rows, L.sh.max_batch, (L.sh.max_batch * seq_rows + 3) / 4});
+  }
+  return (int)std::max<int64_t>(1, std::min<int64_t>(L.grid_merge_cap, wgs));
 }
 
 // The work of a call runs on the device of its stream (the current device
@@ -464,18 +485,8 @@ int launch_all(const Launch& L, const void* q, const void* k_cache, const void* 
     m.part_o = L.part_o;
     m.part_lse = L.part_lse;
     m.hq = L.sh.hq;
-    // Row and head-pair units, one per workgroup (wide) or per wavefront.  A
-    // graph launch gets a workgroup per unit that the query rows of the
-    // latest prepare can need, and loops where a later one needs more (2048
-    // workgroups, mostly idle, took 2 us longer in a decode step of 12
-    // sequences).
-    const int64_t hpairs = (L.sh.hq + 1) / 2;
     m.wide = L.wide_merge[mode] ? 1 : 0;
-    const int64_t wgs = L.graph    ? L.rows * hpairs
-                        : m.wide ? L.n_merge[mode] * hpairs
-                                 : (L.n_merge[mode] * hpairs + 3) / 4;
-    const int grid = (int)std::min<int64_t>(L.grid_merge_cap, wgs);
-    e = launch_merge(m, L.bf16, std::max(grid, 1), st);
+    e = launch_merge(m, L.bf16, merge_grid(L, mode), st);
     if (e != hipSuccess) return hip_fail(e, "merge kernel launch");
   }
   return FE_OK;
@@ -737,7 +748,7 @@ int fe_attn_plan_lists(const fe_attn_plan* p, int causal, int32_t* counts_out) {
   const Launch& L = p->run;
   const int m = causal ? 1 : 0;
   const int32_t counts[] = {L.n_pieces,   L.n_short,  L.n_tile[m], L.tile_rows[m],
-                            L.n_merge[m], L.wide_merge[m] ? 1 : 0, L.tile_stream[m] ? 1 : 0};
+                            L.n_merge[m], L.wide_merge[m] ? 1 : 0, L.tile_stream[m] ? 1 : 0, merge_grid(L, m)};
   std::memcpy(counts_out, counts, sizeof(counts));
   return FE_OK;
 }

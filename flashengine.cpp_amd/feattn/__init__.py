@@ -187,6 +187,7 @@ class PlanLists(NamedTuple):
     merge_rows: int
     merge_wide: int
     tile_stream: int
+    merge_grid: int
 
 
 class Plan:
@@ -218,7 +219,7 @@ class Plan:
 
     def lists(self, causal: bool = True) -> PlanLists:
         """What the latest prepare planned for run(causal=causal) (fe_attn_plan_lists)."""
-        out = (ctypes.c_int32 * 7)()
+        out = (ctypes.c_int32 * 8)()
         _check(lib().fe_attn_plan_lists(self._h, int(bool(causal)), out))
         return PlanLists(*out)
 

@@ -156,11 +156,12 @@ int fe_attn_run_noalloc(const void* q, const void* k_cache, const void* v_cache,
 const char* fe_attn_last_error(void);
 
 /* The work lists of the plan's latest prepare, as fe_attn_run with this
- * `causal` launches them.  counts_out[0..6] = decode items, short-context
+ * `causal` launches them.  counts_out[0..7] = decode items, short-context
  * units (then no decode items), tile items, query rows of a tile item at
  * most, merge rows, form of the merge (0 a wavefront, 1 a workgroup per row
- * and pair of heads), tile reads with the non-temporal hint (0/1).  For
- * callers and tests that want to know which form a batch was given. */
+ * and pair of heads), tile reads with the non-temporal hint (0/1),
+ * workgroups of the merge launch (of a capture made now, for a graph plan).
+ * For callers and tests that want to know which form a batch was given. */
 int fe_attn_plan_lists(const fe_attn_plan* plan, int causal,
                        int32_t* counts_out);
 

@@ -73,3 +73,55 @@ def test_infinite_values_stay_infinite(dev, dtype):
             torch.testing.assert_close(out[~inf], want.float()[~inf], atol=1e-2, rtol=1e-2)
     plan.close()
     graph_plan.close()
+
+
+@pytest.mark.parametrize("hq,hkv,wide_lens,wide_rows,narrow_lens", [(32, 8, [9000, 5000] * 8, 4, [900] * 40),
+                                                                    (5, 5, [1300] * 12, 16, [400, 70, 130] * 13)])
+def test_graph_captured_on_one_short_sequence(dev, hq, hkv, wide_lens, wide_rows, narrow_lens):
+    """A graph captured after a prepare of a single short sequence folds the
+    splits of later, much larger batches: more rows and head pairs than the
+    launch has workgroups for in the wide form (so workgroups take several),
+    and the narrow one; every replay against the oracle and the bits of an
+    eager plan."""
+    blocks, batch, hpairs = 8000, 40, (hq + 1) // 2
+    max_pages = 9000 // 16 + 3
+    plan = feattn.Plan(hq, hkv, 128, 16, batch, max_pages, True, blocks)
+    eager = feattn.Plan(hq, hkv, 128, 16, batch, max_pages, True, blocks)
+    one = W.make_batch(hq, hkv, starts=[30], qlens=[1], seed=1, pool=blocks)
+    plan.prepare(one.qo, one.kv, one.pages, one.last, one.batch, one.rows, graph=True)
+    grid = plan.lists().merge_grid
+    assert grid >= batch * hpairs  # one pass for every row of a batch of the plan's size
+    assert grid < len(wide_lens) * wide_rows * hpairs  # several for these rows
+    gen = torch.Generator().manual_seed(3)
+    kc = torch.randn(blocks + 1, 16, hkv, 128, generator=gen).to(torch.bfloat16)
+    vc = torch.randn(blocks + 1, 16, hkv, 128, generator=gen).to(torch.bfloat16)
+    kd, vd = kc.to(dev), vc.to(dev)
+    q = torch.zeros(16 * batch, hq, 128, dtype=torch.bfloat16, device=dev)
+    out = torch.zeros_like(q)
+    lse = torch.zeros(16 * batch, hq, device=dev)
+    graph = torch.cuda.CUDAGraph()
+    torch.cuda.synchronize()
+    with torch.cuda.graph(graph):
+        plan.run(q, kd, vd, out, causal=True, lse=lse)
+    for wide, lens, rows in ((1, wide_lens, wide_rows), (0, narrow_lens, 1), (1, wide_lens, 1), (0, [40, 50], 1),
+                             (1, wide_lens, wide_rows)):
+        b = W.make_batch(hq, hkv, starts=[n - rows for n in lens], qlens=[rows] * len(lens), seed=len(lens),
+                         pool=blocks)
+        qb = torch.randn(b.rows, hq, 128, generator=gen).to(torch.bfloat16)
+        q[:b.rows].copy_(qb)
+        out.fill_(float("nan"))
+        lse.fill_(float("nan"))
+        plan.prepare(b.qo, b.kv, b.pages, b.last, b.batch, b.rows, graph=True)
+        eager.prepare(b.qo, b.kv, b.pages, b.last, b.batch, b.rows)
+        forms = plan.lists()
+        assert forms.merge_wide == wide and (forms.merge_rows > 0 or lens == [40, 50])
+        graph.replay()
+        o2, l2 = torch.zeros_like(q[:b.rows]), torch.zeros_like(lse[:b.rows])
+        eager.run(q, kd, vd, o2, causal=True, lse=l2)
+        torch.cuda.synchronize()
+        want, want_lse = A.run(b, qb, kc, vc, True)
+        torch.testing.assert_close(o2.float().cpu(), want.float(), atol=1e-2, rtol=1e-2)
+        torch.testing.assert_close(l2.cpu(), want_lse, atol=1e-3, rtol=0)
+        assert torch.equal(out[:b.rows], o2) and torch.equal(lse[:b.rows], l2)
+    plan.close()
+    eager.close()
