@@ -336,16 +336,17 @@ void init_launch(Launch& L, const PlanShape& sh, bool bf16) {
   L.grid_merge_cap = sh.num_cus * 8;
 }
 
-// Launch sizes of the lists just staged.
-// Whether the tile lists read each K/V token once per kv head: no sequence
-// with tile work is cut into several column blocks (the planner gives such a
-// sequence ceil(qlen / tile_rows) blocks, every one over the same tokens).  Chunked prefill is cut so, and those re-reads are L2 hits with
-// the default policy (the 8192-token prefill takes 0.257 ms so, 0.282 ms
-// streamed); DFlash blocks and short verify rows are one block each.
-bool reads_tokens_once(const BuiltPlan& bp, const PlanShape& sh, int mode) {
+// Whether tile lists of items of at most `item_rows` query rows read each K/V
+// token once per kv head: no sequence with tile work is cut into several
+// column blocks (the planner gives such a sequence ceil(qlen / item_rows)
+// blocks, every one over the same tokens).  Chunked prefill is cut so, and
+// those re-reads are L2 hits with the default policy (the 8192-token prefill
+// takes 0.257 ms so, 0.282 ms streamed); DFlash blocks and short verify rows
+// are one block each.
+bool reads_tokens_once(const BuiltPlan& bp, const PlanShape& sh, int item_rows) {
   const int group = sh.hq / sh.hkv;
   for (const SeqInfo& s : bp.seqs)
-    if (s.qlen * group > kDecodeCols && s.qlen > bp.mode[mode].tile_rows) return false;
+    if (s.qlen * group > kDecodeCols && s.qlen > item_rows) return false;
   return true;
 }
 
@@ -356,6 +357,7 @@ int short_waves(const PlanShape& sh) {
   return w >= kShortMinWaves ? w : 0;
 }
 
+// Launch sizes of the lists just staged.
 void record_lists(Launch& L, const BuiltPlan& bp, const HeapPlace& hp, int nc) {
   L.rows = 0;
   for (const SeqInfo& s : bp.seqs) L.rows += s.qlen;
@@ -371,10 +373,14 @@ void record_lists(Launch& L, const BuiltPlan& bp, const HeapPlace& hp, int nc) {
     L.n_merge[m] = (int)bp.mode[m].merge.size();
     L.wide_merge[m] = merge_wide(bp.mode[m].merge, L.sh);
     // Graph plans keep the policy their tile launch was captured with (a
-    // cache hint: results do not depend on it).
-    const bool once = reads_tokens_once(bp, L.sh, m);
-    if (L.graph && L.graph_stream[m] < 0) L.graph_stream[m] = once ? 1 : 0;
-    L.tile_stream[m] = L.graph ? L.graph_stream[m] > 0 : once;
+    // cache hint: results do not depend on it): the full-width items', also
+    // where the first batch is small and has half-width ones, since later ones
+    // may be long (captured on 1 x 16 over 100, 32/4 heads, and replayed on 32 x
+    // 16 over 12000: 147 us, 165 without the hint; on 8 x 16 over 300: 12.5 and
+    // 12.4).
+    if (L.graph && L.graph_stream[m] < 0)
+      L.graph_stream[m] = reads_tokens_once(bp, L.sh, kTileCols / (L.sh.hq / L.sh.hkv)) ? 1 : 0;
+    L.tile_stream[m] = L.graph ? L.graph_stream[m] > 0 : reads_tokens_once(bp, L.sh, bp.mode[m].tile_rows);
   }
 }
 

@@ -190,3 +190,26 @@ def test_small_tile_items(dev, hq, hkv, starts, qlens, dtype, causal):
         torch.testing.assert_close(lse.cpu(), want_lse, atol=1e-3, rtol=0)
         got.append((out, lse))
     assert torch.equal(got[0][0], got[1][0]) and torch.equal(got[0][1], got[1][1])
+
+
+@pytest.mark.gpu
+def test_graph_tile_policy_is_the_full_width_items(dev):
+    """Short 16-row blocks of 8 heads per kv head are planned as half-width
+    items, whose second block reads the K/V again; long ones are one item
+    each.  A graph plan's cache policy is fixed by its first prepare, and that
+    of the long ones whichever comes first; an eager plan follows each batch."""
+    short = W.make_batch(32, 4, starts=[100, 60], qlens=[16, 16], seed=1, pool=2000)
+    long = W.make_batch(32, 4, starts=[9000, 12000], qlens=[16, 16], seed=2, pool=2000)
+    chunk = W.make_batch(32, 4, starts=[0, 30], qlens=[200, 16], seed=2, pool=2000)
+    want = {id(short): (8, 0), id(long): (16, 1), id(chunk): (8, 0)}
+    for first, policy in ((short, 1), (long, 1), (chunk, 0)):
+        plan = feattn.Plan(32, 4, 128, 16, 2, 800, True, 2000)
+        for b in (first, short, long, chunk):
+            plan.prepare(b.qo, b.kv, b.pages, b.last, b.batch, b.rows, graph=True)
+            for causal in (True, False):
+                got = plan.lists(causal)
+                assert (got.tile_rows, got.tile_stream) == (want[id(b)][0], policy)
+        for b in (short, long, chunk):
+            plan.prepare(b.qo, b.kv, b.pages, b.last, b.batch, b.rows)
+            assert (plan.lists().tile_rows, plan.lists().tile_stream) == want[id(b)]
+        plan.close()
