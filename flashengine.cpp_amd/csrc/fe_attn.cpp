@@ -508,7 +508,8 @@ int report_error(int code, const std::string& msg) { return fail(code, msg); }
 // One-shot attention whose metadata arena and split-KV partials are carved
 // out of `arena` (`bytes` of device memory on `device`): plans exactly as
 // fe_attn_plan_prepare does for a plan of the same heads, page and blocks
-// (so the results are identical), stages the metadata with one copy on `st`
+// (so the results are identical, but for a call that the arena only holds in
+// the general form of its lists), stages the metadata with one copy on `st`
 // and launches as fe_attn_run does.  Allocates no device or pinned memory.
 int attn_oneshot(uint8_t* arena, size_t bytes, int device, const void* q, const void* k_cache, const void* v_cache,
                  void* out, float* lse, int causal, const int32_t* qo, const int32_t* kv, const int32_t* pages,
@@ -544,24 +545,32 @@ int attn_oneshot(uint8_t* arena, size_t bytes, int device, const void* q, const 
   rc = check_stream_device(st, device);
   if (rc != FE_OK) return rc;
   BuiltPlan bp;
-  rc = build_plan(sh, qo, kv, pages, last, batch, rows, bp, err, short_waves(sh), true);
-  if (rc != FE_OK) return fail(rc, err);
   const int mode = causal ? 1 : 0;
   const int npages = batch > 0 ? kv[batch] : 0;
   const bool staged[2] = {mode == 0, mode == 1};
-  const HeapPlace hp = place_lists(bp, npages, staged);
-  Regions r{};
-  r.seqs = bp.seqs.size();
-  r.tshare[mode] = (size_t)sh.tile_slots + 1;
-  r.shares = (size_t)share_cap(sh);
-  r.heap = hp.used;
   Launch L;
   init_launch(L, sh, bf16 != 0);
-  L.lay = make_layout(r);
-  const size_t parts = (size_t)bp.mode[mode].partial_rows * hq;
-  const size_t o_off = L.lay.total;
-  const size_t lse_off = align256(o_off + parts * kHeadDim * sizeof(uint16_t));
-  const size_t need = lse_off + parts * sizeof(float);
+  HeapPlace hp;
+  size_t o_off = 0, lse_off = 0, need = 0;
+  // The forms for small calls take up to 128 bytes a sequence and 32 an item
+  // more than the general plan where that splits nothing: a call that only
+  // fits in the general form is planned so.
+  for (const bool forms : {true, false}) {
+    rc = build_plan(sh, qo, kv, pages, last, batch, rows, bp, err, forms ? short_waves(sh) : 0, forms);
+    if (rc != FE_OK) return fail(rc, err);
+    hp = place_lists(bp, npages, staged);
+    Regions r{};
+    r.seqs = bp.seqs.size();
+    r.tshare[mode] = (size_t)sh.tile_slots + 1;
+    r.shares = (size_t)share_cap(sh);
+    r.heap = hp.used;
+    L.lay = make_layout(r);
+    const size_t parts = (size_t)bp.mode[mode].partial_rows * hq;
+    o_off = L.lay.total;
+    lse_off = align256(o_off + parts * kHeadDim * sizeof(uint16_t));
+    need = lse_off + parts * sizeof(float);
+    if (need <= bytes) break;
+  }
   if (need > bytes)
     return fail(FE_ECAPACITY, "attention (no-alloc): this call needs " + std::to_string(need) +
                                   " bytes of device scratch, more than the " + std::to_string(bytes) + " it holds");

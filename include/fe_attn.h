@@ -124,16 +124,18 @@ int fe_rope_append(void* q, const void* k, const void* v, void* k_cache,
 
 /* No counterpart in the reference.  For callers that cannot allocate device
  * memory (serving loops and harnesses that forbid hipMalloc):
- * fe_attn_plan_prepare + fe_attn_run in one call, without a plan.  Same arguments and results as a plan of (hq, hkv, dim, page,
- * blocks, bf16) prepared with (qo, kv, pages, last, batch, rows) and run
+ * fe_attn_plan_prepare + fe_attn_run in one call, without a plan.  Same
+ * arguments and results as a plan of (hq, hkv, dim, page, blocks, bf16)
+ * prepared with (qo, kv, pages, last, batch, rows) and run
  * with (q, k_cache, v_cache, out, lse, causal): the same work lists, kernels
- * and bits.  The work lists and split-KV partials live in a 48 MiB device
+ * and bits (a small call whose page table leaves room only for the general
+ * plan's lists is run in that form).  The work lists and split-KV partials live in a 48 MiB device
  * array of the library (one per device, reserved when the library's code
  * object loads on that device, whether or not this entry point is ever
  * called, and kept until the process ends): enough for the full split-KV
  * budget of any plan with up to 128 query heads plus 15.5 MiB of work lists
- * and page table; a call that needs more returns FE_ECAPACITY.  Allocates no device or pinned
- * memory; the metadata goes to the device by one copy from pageable host
+ * and page table; a call that needs more returns FE_ECAPACITY.  Allocates no
+ * device or pinned memory; the metadata goes to the device by one copy from pageable host
  * memory on `stream`, which HIP performs synchronously: the call returns
  * after the stream's earlier work and the copy have run.  For the same
  * reason it cannot be captured into a HIP graph (a replay would copy from

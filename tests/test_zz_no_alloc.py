@@ -111,6 +111,42 @@ def test_noalloc_rejects_calls_beyond_its_scratch(dev):
     assert torch.isnan(out.float()).all()
 
 
+def test_noalloc_small_call_at_the_scratch_limit(dev):
+    """A batch of 64 short sequences whose page table stands behind millions
+    of entries of other sequences: where the short-context records no longer
+    fit the scratch but the general plan's smaller lists do, the call still
+    runs (checked against the call without the offset, 16-bit outputs, within
+    their rounding), and past that it is refused."""
+    b = W.make_batch(32, 8, starts=[63] * 64, qlens=[1] * 64, seed=5)
+    q, kc, vc = (t.to(dev) for t in W.make_tensors(b, seed=5))
+    want = torch.full_like(q, float("nan"))
+    feattn.run_noalloc(q, kc, vc, want, b.qo, b.kv, b.pages, b.last, b.batch, b.rows, 32, 8, 128, 16, b.blocks, True)
+
+    def call(offset, out):
+        pages = np.zeros(offset + len(b.pages), dtype=np.int32)
+        pages[offset:] = b.pages
+        feattn.run_noalloc(q, kc, vc, out, b.qo, [offset + k for k in b.kv],
+                           (ctypes.c_int32 * len(pages)).from_buffer(pages), b.last, b.batch, b.rows, 32, 8, 128, 16,
+                           b.blocks, True)
+
+    far = 13_000_000
+    out = torch.full_like(q, float("nan"))
+    with pytest.raises(RuntimeError, match="scratch") as refused:
+        call(far, out)
+    need, held = (int(w) for w in str(refused.value).replace(",", "").split() if w.isdigit() and len(w) > 5)
+    # 16-byte sequence and 32-byte piece records, share records and offsets of
+    # 256 compute units; short-context records take 160 bytes a sequence
+    assert need - 4 * (far + len(b.pages)) < 64 * (16 + 32) + 256 * 64 + 4 * 513 + 6 * 256
+    limit = far - (need - held + 3) // 4 // 64 * 64 - 64  # an offset the general lists fit at, by at most 512 bytes
+    with pytest.raises(RuntimeError, match="scratch"):
+        call(limit + 256, out)
+    torch.cuda.synchronize()
+    assert torch.isnan(out.float()).all()
+    call(limit, out)
+    torch.cuda.synchronize()
+    torch.testing.assert_close(out.float(), want.float(), atol=1e-2, rtol=1e-2)
+
+
 def test_noalloc_rejects_bad_arguments(dev):
     """The plan entry points' checks hold without a plan: head size,
     alignment, negative batch and invalid metadata are refused on the host
