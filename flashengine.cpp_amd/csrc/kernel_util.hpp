@@ -41,59 +41,52 @@ __device__ __forceinline__ SeqInfo ldc_seq(const SeqInfo* seqs, int i) {
   return SeqInfo{ldc(p, 0), ldc(p, 1), ldc(p, 2), ldc(p, 3)};
 }
 
+// 16 bytes per lane from global memory to LDS (lane i's at lds_addr + 16 i).
+// m0 holds the LDS address; the instruction needs a wait state after m0's
+// write.
+__device__ __forceinline__ void lds_dma16(const void* gaddr, uint32_t lds_addr) {
+  asm volatile(
+      "s_mov_b32 m0, %1\n\t"
+      "s_nop 0\n\t"
+      "global_load_lds_dwordx4 %0, off"
+      :
+      : "v"(gaddr), "s"(__builtin_amdgcn_readfirstlane(lds_addr))  // wave-uniform by construction
+      : "memory", "m0");
+}
+
+// The same from a wave-uniform base and a 32-bit byte offset per lane: no
+// 64-bit address per lane to compute.  A base that the vector unit has just
+// written (readfirstlane, a lane reload of a spilled register) needs five wait
+// states before a memory instruction reads it, and the compiler does not look
+// into the asm for them: the scalar unit, which waits by itself, copies it, in
+// the wait state that m0 needs.  (Wait states instead, or the four copies of a
+// block in one asm with a single run of them: 8192-token prefill +0.3 %, 777
+// tokens +0.5 %.)
+//
 // STREAM: the non-temporal hint, for data that no other work of the launch
 // reads again (K/V rows streamed once).  Such reads then neither displace
 // reused lines nor cost cache allocation on their way: the decode kernel
 // streams 6.4-6.9 TB/s with it against 5.7-6.1 without.
 template <bool STREAM = false>
-__device__ __forceinline__ void lds_dma16(const void* gaddr, uint32_t lds_addr) {
-  uint32_t saved;
-  if constexpr (STREAM) {
-    asm volatile(
-        "s_mov_b32 %0, m0\n\t"
-        "s_mov_b32 m0, %2\n\t"
-        "s_nop 0\n\t"
-        "global_load_lds_dwordx4 %1, off nt\n\t"
-        "s_mov_b32 m0, %0"
-        : "=&s"(saved)
-        : "v"(gaddr), "s"(__builtin_amdgcn_readfirstlane(lds_addr))  // wave-uniform by construction
-        : "memory");
-  } else {
-    asm volatile(
-        "s_mov_b32 %0, m0\n\t"
-        "s_mov_b32 m0, %2\n\t"
-        "s_nop 0\n\t"
-        "global_load_lds_dwordx4 %1, off\n\t"
-        "s_mov_b32 m0, %0"
-        : "=&s"(saved)
-        : "v"(gaddr), "s"(__builtin_amdgcn_readfirstlane(lds_addr))  // wave-uniform by construction
-        : "memory");
-  }
-}
-
-// The same from a wave-uniform base and a 32-bit byte offset per lane: no
-// 64-bit address per lane to compute.  m0 is not saved: gfx9's LDS
-// instructions do not read it, and the compiler holds no value there (it
-// writes m0 right before an instruction of its own that reads it).
-template <bool STREAM = false>
 __device__ __forceinline__ void lds_dma16(const char* base, uint32_t off, uint32_t lds_addr) {
   const uint32_t m = __builtin_amdgcn_readfirstlane(lds_addr);
+  const char* copy;
   if constexpr (STREAM) {
     asm volatile(
-        "s_mov_b32 m0, %1\n\t"
-        "s_nop 0\n\t"
-        "global_load_lds_dwordx4 %0, %2 nt"
-        :
+        "s_mov_b32 m0, %2\n\t"
+        "s_mov_b64 %0, %3\n\t"
+        "global_load_lds_dwordx4 %1, %0 nt"
+        : "=&s"(copy)
         : "v"(off), "s"(m), "s"(base)
-        : "memory");
+        : "memory", "m0");
   } else {
     asm volatile(
-        "s_mov_b32 m0, %1\n\t"
-        "s_nop 0\n\t"
-        "global_load_lds_dwordx4 %0, %2"
-        :
+        "s_mov_b32 m0, %2\n\t"
+        "s_mov_b64 %0, %3\n\t"
+        "global_load_lds_dwordx4 %1, %0"
+        : "=&s"(copy)
         : "v"(off), "s"(m), "s"(base)
-        : "memory");
+        : "memory", "m0");
   }
 }
 
