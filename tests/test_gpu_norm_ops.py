@@ -52,8 +52,9 @@ def test_norm_bit_exact(dev, bf16, width, residual):
 
 @pytest.mark.parametrize("bf16", [True, False])
 @pytest.mark.parametrize("width,offset", [(8, 0), (248, 0), (256, 0), (264, 0), (504, 0), (520, 0), (1024, 0),
-                                          (1032, 0), (3064, 0), (6144, 0), (8192, 0), (8200, 0), (1, 0), (257, 0),
-                                          (1022, 0), (3001, 0), (6145, 0), (512, 1), (4096, 4)])
+                                          (1032, 0), (2048, 0), (3064, 0), (3840, 0), (4096, 0), (4104, 0), (5120, 0),
+                                          (6144, 0), (8192, 0), (8200, 0), (1, 0), (257, 0), (1022, 0), (3001, 0),
+                                          (6145, 0), (512, 1), (4096, 4)])
 def test_norm_widths_and_alignments(dev, bf16, width, offset):
     """Bit-exact on both sides of every stripe, pair and register bound of the
     kernels, on widths that are no multiple of a load and on tensors that
@@ -101,23 +102,53 @@ def test_norm_widths_and_alignments(dev, bf16, width, offset):
 
 
 @pytest.mark.parametrize("bf16", [True, False])
-def test_norm_large_call_equals_small_calls(dev, bf16):
+@pytest.mark.parametrize("rows,width", [(2051, 2048), (1031, 4096), (1031, 5120), (1031, 8192), (4099, 128 * 9)])
+@pytest.mark.parametrize("residual", [True, False])
+def test_norm_large_call_equals_small_calls(dev, bf16, rows, width, residual):
     """A call past the L2's size streams its tensors; every row's bits are
-    those of the same rows in small calls (the last one, of an odd count)."""
-    rows, width = 2051, 2048
+    those of the same rows in small calls (the last one, of an odd count).
+    Then the large call in place, x and the residual overwritten."""
+    rows = rows if residual else 2 * rows - 1
+    assert rows * width * (8 if residual else 4) >= 32 << 20
     gen = torch.Generator(device=dev).manual_seed(5)
     x = (torch.randn(rows, width, generator=gen, device=dev) * 3).to(dtype_of(bf16))
-    r = torch.randn(rows, width, generator=gen, device=dev).to(x.dtype)
+    r = torch.randn(rows, width, generator=gen, device=dev).to(x.dtype) if residual else None
     w = (1 + 0.1 * torch.randn(width, generator=gen, device=dev)).to(x.dtype)
-    out, new = torch.empty_like(x), torch.empty_like(x)
+    out, part = torch.empty_like(x), torch.empty_like(x)
+    new, part_new = (torch.empty_like(x), torch.empty_like(x)) if residual else (None, None)
     feattn.norm(x, w, out, rows, width, 1e-6, bf16, residual=r, new_residual=new)
-    part, part_new = torch.empty_like(x), torch.empty_like(x)
     for i in range(0, rows, 300):
         n = min(300, rows - i)
-        feattn.norm(x[i:], w, part[i:], n, width, 1e-6, bf16, residual=r[i:], new_residual=part_new[i:])
+        feattn.norm(x[i:], w, part[i:], n, width, 1e-6, bf16, residual=None if r is None else r[i:],
+                    new_residual=None if new is None else part_new[i:])
+    feattn.norm(x, w, x, rows, width, 1e-6, bf16, residual=r, new_residual=r)
     torch.cuda.synchronize()
     assert torch.equal(out.view(torch.int16), part.view(torch.int16))
-    assert torch.equal(new.view(torch.int16), part_new.view(torch.int16))
+    assert torch.equal(out.view(torch.int16), x.view(torch.int16))
+    if residual:
+        assert torch.equal(new.view(torch.int16), part_new.view(torch.int16))
+        assert torch.equal(new.view(torch.int16), r.view(torch.int16))
+
+
+@pytest.mark.parametrize("bf16", [True, False])
+@pytest.mark.parametrize("width", [128, 4096, 5120, 8192])
+def test_norm_in_place_many_rows(dev, bf16, width):
+    """x and the residual overwritten by a call of more rows than the block
+    kernel takes (and less than what streams): the oracle's bits."""
+    gen = torch.Generator().manual_seed(width)
+    rows, reps = 4, 130
+    x = (torch.randn(rows, width, generator=gen) * 3).to(dtype_of(bf16))
+    r = torch.randn(rows, width, generator=gen).to(x.dtype)
+    w = (1 + 0.1 * torch.randn(width, generator=gen)).to(x.dtype)
+    want, want_res = N.rms_norm(u16(x), u16(w), 1e-6, bf16, residual=u16(r))
+    plain, _ = N.rms_norm(u16(x), u16(w), 1e-6, bf16, residual=None)
+    xd, rd, yd = x.repeat(reps, 1).to(dev), r.repeat(reps, 1).to(dev), x.repeat(reps, 1).to(dev)
+    feattn.norm(xd, w.to(dev), xd, rows * reps, width, 1e-6, bf16, residual=rd, new_residual=rd)
+    feattn.norm(yd, w.to(dev), yd, rows * reps, width, 1e-6, bf16)
+    torch.cuda.synchronize()
+    for got, ref in ((xd, want), (rd, want_res), (yd, plain)):
+        got = u16(got).reshape(reps, rows, width)
+        assert np.array_equal(got, np.broadcast_to(ref, got.shape))
 
 
 def make_fused_case(bf16, rows, hq, hkv, row_stride, seed, cache_pages=64, max_pos=4096):

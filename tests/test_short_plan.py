@@ -213,3 +213,45 @@ def test_graph_tile_policy_is_the_full_width_items(dev):
             plan.prepare(b.qo, b.kv, b.pages, b.last, b.batch, b.rows)
             assert (plan.lists().tile_rows, plan.lists().tile_stream) == want[id(b)]
         plan.close()
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("hq,hkv,seqs,hi", [(32, 8, 64, 128), (32, 4, 200, 64), (8, 8, 64, 100)])
+@pytest.mark.parametrize("dtype", ["bf16", "f16"])
+def test_graph_workgroups_take_several_short_units(dev, hq, hkv, seqs, hi, dtype):
+    """More short-context units than a graph's launch has workgroups, so each
+    takes a second one in the same LDS; captured on a single sequence, replayed
+    on batches of this size, a smaller one and this again, against the oracle
+    and the bits of an eager plan (one unit per workgroup)."""
+    blocks = seqs * (hi // 16 + 1) + 2
+    plan, eager = (feattn.Plan(hq, hkv, 128, 16, seqs, hi // 16 + 3, dtype == "bf16", blocks) for _ in range(2))
+    one = W.make_batch(hq, hkv, starts=[20], qlens=[1], seed=1, pool=blocks)
+    plan.prepare(one.qo, one.kv, one.pages, one.last, one.batch, one.rows, graph=True)
+    q, kc, vc = W.make_tensors(W.make_batch(hq, hkv, starts=[hi - 1] * seqs, qlens=[1] * seqs, seed=2, pool=blocks),
+                               seed=3, dtype=dtype)
+    qd, kd, vd = q.to(dev), kc.to(dev), vc.to(dev)
+    out, lse = torch.zeros_like(qd), torch.zeros(seqs, hq, device=dev)
+    graph = torch.cuda.CUDAGraph()
+    torch.cuda.synchronize()
+    with torch.cuda.graph(graph):
+        plan.run(qd, kd, vd, out, causal=True, lse=lse)
+    cus = torch.cuda.get_device_properties(dev).multi_processor_count
+    for i, n in enumerate((seqs, 3, seqs, seqs)):
+        b = W.make_batch(hq, hkv, starts=[(37 * s + 5 * i) % hi for s in range(n)], qlens=[1] * n, seed=4 + i,
+                         pool=blocks)
+        plan.prepare(b.qo, b.kv, b.pages, b.last, b.batch, b.rows, graph=True)
+        eager.prepare(b.qo, b.kv, b.pages, b.last, b.batch, b.rows)
+        units = plan.lists().short_units
+        assert units == n * hkv and (n == 3 or units > cus * 8 // hkv)  # the launch: 8 wavefronts per CU
+        out.fill_(float("nan"))
+        lse.fill_(float("nan"))
+        graph.replay()
+        o2, l2 = torch.zeros_like(qd[:n]), torch.zeros_like(lse[:n])
+        eager.run(qd, kd, vd, o2, causal=True, lse=l2)
+        torch.cuda.synchronize()
+        want, want_lse = A.run(b, q[:n], kc, vc, True)
+        torch.testing.assert_close(o2.float().cpu(), want.float(), atol=1e-2, rtol=1e-2)
+        torch.testing.assert_close(l2.cpu(), want_lse, atol=1e-3, rtol=0)
+        assert torch.equal(out[:n], o2) and torch.equal(lse[:n], l2)
+    plan.close()
+    eager.close()
