@@ -214,8 +214,12 @@ bool cut_tile_stream(const std::vector<SeqInfo>& seqs, int G, int hkv, bool caus
 //     x 1001 whole, cut 12.2.
 //   * cut into steps: 13.7 / 18.3 (1 x 4001), 13.8 / 17.4 (4 x 1984).
 //   * more items than resident workgroups: 17.0 / 15.9 (64 x 200) and, cut,
-//     27.9 / 22.3 (12 x 2048); only sequences of one block per wavefront
-//     still gain, 12.1 / 14.6 (64 x 64).
+//     27.9 / 22.3 (12 x 2048); up to twice as many still gain where no sequence
+//     is longer than 64 tokens, 11.4 / 15.1 (64 x 41), 13.5 / 15.5 (200 x 33, W =
+//     4), in a graph 13.3 / 15.0 and 15.7 / 15.4 -- but only against a merge:
+//     where every sequence lies within one share, 12.4 / 9.9 (64 x 64), 15.6 /
+//     10.2 (200 x 64, W = 4); and not longer ones, 17.0 / 13.2 (64 x 128), in a
+//     graph 18.9 / 13.1.
 //   * with more K and V per compute unit, the shares' whole-page streams win
 //     when the cache is cold: 188 KB, inside a replayed decode step, 1.6 us a
 //     layer slower so.  Two column blocks are slow on the shares (20.3 /
@@ -226,6 +230,8 @@ bool plan_short(const PlanShape& sh, const int32_t* pages, int waves, BuiltPlan&
   const int step = 64 * waves;
   int max_len = 0, max_cols = 0;
   int64_t whole = 0, cut = 0, tokens = 0;  // items of either form
+  int64_t off = 0;                         // in the stream of the decode shares
+  bool crossing = false;                   // a sequence crosses the border of two (shortest) shares
   for (const SeqInfo& s : out.seqs) {
     if (s.qlen == 0) continue;
     if (s.qlen * G > kDecodeCols) return false;
@@ -234,13 +240,17 @@ bool plan_short(const PlanShape& sh, const int32_t* pages, int waves, BuiltPlan&
     whole += sh.hkv;
     cut += (int64_t)sh.hkv * ceil_div(s.len, step);
     tokens += s.len;
+    const int64_t end = off + round_up(s.len, 16);
+    crossing = crossing || off / kMinShareTokens != (end - 1) / kMinShareTokens;
+    off = end;
   }
   if (whole == 0) return false;
   const int64_t per_cu = tokens * sh.hkv * (2 * kHeadDim * 2) / sh.num_cus;
   const int64_t limit = max_cols <= 16 ? 144 << 10 : 256 << 10;
   if (per_cu > limit) return false;
   int piece;
-  if (max_len <= 512 && (whole <= slots || (max_len <= 16 * waves && whole <= 2 * slots)))
+  // (Twice as many workgroups of such sequences: the shares are the shortest.)
+  if (max_len <= 512 && (whole <= slots || (max_len <= kMinShareTokens && whole <= 2 * slots && crossing)))
     piece = 512;
   else if (cut <= slots)
     piece = step;

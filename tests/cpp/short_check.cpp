@@ -223,7 +223,46 @@ static bool check_prompts(int hq, int hkv, int& ordinary) {
   return true;
 }
 
+// Decode batches of one length, up to and past the workgroups that run at
+// once: beyond them only sequences of at most 64 tokens that the shares would
+// have to merge are short-context items.
+static bool check_two_sets() {
+  for (const int waves : {4, 8})
+    for (const int len : {16, 30, 33, 48, 49, 64, 65, 100, 128}) {
+      Case c;
+      c.sh.hq = 32;
+      c.sh.hkv = waves;
+      c.sh.dim = 128;
+      c.sh.page = 16;
+      c.sh.max_pages = 10;
+      c.sh.partial_cap = 8192;
+      const int slots = c.sh.decode_waves / waves / waves;  // sequences whose workgroups run at once
+      for (const int seqs : {slots, slots + 1, 2 * slots, 2 * slots + 1}) {
+        const int np = (len + 15) / 16;
+        c.sh.max_batch = seqs;
+        c.sh.blocks = seqs * np;
+        c.qo.assign(1, 0);
+        c.kv.assign(1, 0);
+        c.pages.clear();
+        c.last.assign(seqs, len - 16 * (np - 1));
+        for (int b = 0; b < seqs; ++b) {
+          c.qo.push_back(b + 1);
+          c.kv.push_back((b + 1) * np);
+          for (int i = 0; i < np; ++i) c.pages.push_back(b * np + i);
+        }
+        BuiltPlan bp;
+        std::string err;
+        CHECK(build_plan(c.sh, c.qo.data(), c.kv.data(), c.pages.data(), c.last.data(), seqs, seqs, bp, err, waves) ==
+              FE_OK);
+        const bool merged = np == 3;  // 48-token strides cross the shares' 64-token borders
+        CHECK(!bp.shorts.empty() == (seqs <= slots || (seqs <= 2 * slots && len <= 64 && merged)));
+      }
+    }
+  return true;
+}
+
 int main() {
+  if (!check_two_sets()) return 1;
   static const int heads[][2] = {{4, 1},  {8, 2},  {8, 8},  {12, 2}, {16, 2}, {16, 8},
                                  {28, 4}, {32, 4}, {32, 8}, {40, 8}, {64, 4}, {64, 8}};
   for (const auto& h : heads) {

@@ -216,7 +216,7 @@ def test_graph_tile_policy_is_the_full_width_items(dev):
 
 
 @pytest.mark.gpu
-@pytest.mark.parametrize("hq,hkv,seqs,hi", [(32, 8, 64, 128), (32, 4, 200, 64), (8, 8, 64, 100)])
+@pytest.mark.parametrize("hq,hkv,seqs,hi", [(32, 8, 64, 64), (32, 4, 200, 64), (8, 8, 50, 60)])
 @pytest.mark.parametrize("dtype", ["bf16", "f16"])
 def test_graph_workgroups_take_several_short_units(dev, hq, hkv, seqs, hi, dtype):
     """More short-context units than a graph's launch has workgroups, so each
