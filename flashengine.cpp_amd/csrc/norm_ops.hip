@@ -483,10 +483,19 @@ static hipError_t norm_launch(const uint16_t* x, const uint16_t* res, const uint
   auto go = [&](auto kernel) {
     hipLaunchKernelGGL(kernel, dim3(rows), dim3(256), 0, st, x, res, w, out, new_res, width, eps);
   };
-  if (stripes <= 4) go(norm_block_kernel<BF16, 4>);
+  // One stripe: 8192 rows of 11 take 6.2 us with one kept, 7.6 with four.  Rows
+  // of more stripes than can be kept: while their blocks are all resident (768)
+  // what counts are the loads in flight, 600 x 16384 34.3 us with 24 kept, 45.1
+  // with 8; many rows need the wavefronts that fewer registers leave room for,
+  // the more the longer what is read twice: 2000 x 16384 90.9 and 56.3, 800 x
+  // 12288 39.7 and 36.2, but 800 x 9984 28.5 and 28.8, 1600 x 9984 39.0 and 34.5,
+  // 3000 x 8704 44.9 and 48.7.
+  if (stripes <= 1) go(norm_block_kernel<BF16, 1>);
+  else if (stripes <= 4) go(norm_block_kernel<BF16, 4>);
   else if (stripes <= 8) go(norm_block_kernel<BF16, 8>);
   else if (stripes <= 16) go(norm_block_kernel<BF16, 16>);
-  else go(norm_block_kernel<BF16, 24>);
+  else if (stripes <= 34 || rows <= (stripes < 48 ? 1536 : 768)) go(norm_block_kernel<BF16, 24>);
+  else go(norm_block_kernel<BF16, 8>);
   return hipGetLastError();
 }
 

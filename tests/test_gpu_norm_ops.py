@@ -151,6 +151,29 @@ def test_norm_in_place_many_rows(dev, bf16, width):
         assert np.array_equal(got, np.broadcast_to(ref, got.shape))
 
 
+@pytest.mark.parametrize("bf16", [True, False])
+@pytest.mark.parametrize("rows,width,residual", [(600, 9001, True), (1540, 9001, True), (1537, 9984, False),
+                                                 (770, 12288, True), (769, 16384, False), (513, 16391, True),
+                                                 (1030, 33 * 256, True)])
+def test_norm_wide_rows(dev, bf16, rows, width, residual):
+    """Rows of more stripes than the block kernel keeps, on both sides of the
+    row counts where it keeps fewer; the same few rows again and again."""
+    gen = torch.Generator().manual_seed(width)
+    reps = -(-rows // 3)
+    x = (torch.randn(3, width, generator=gen) * 3).to(dtype_of(bf16))
+    r = torch.randn(3, width, generator=gen).to(x.dtype) if residual else None
+    w = (1 + 0.1 * torch.randn(width, generator=gen)).to(x.dtype)
+    want, want_res = N.rms_norm(u16(x), u16(w), 1e-6, bf16, residual=u16(r) if residual else None)
+    xd = x.repeat(reps, 1)[:rows].to(dev)
+    rd = r.repeat(reps, 1)[:rows].to(dev) if residual else None
+    out, new = torch.empty_like(xd), torch.empty_like(xd) if residual else None
+    feattn.norm(xd, w.to(dev), out, rows, width, 1e-6, bf16, residual=rd, new_residual=new)
+    torch.cuda.synchronize()
+    assert np.array_equal(u16(out), np.tile(want, (reps, 1))[:rows])
+    if residual:
+        assert np.array_equal(u16(new), np.tile(want_res, (reps, 1))[:rows])
+
+
 def make_fused_case(bf16, rows, hq, hkv, row_stride, seed, cache_pages=64, max_pos=4096):
     dt = dtype_of(bf16)
     gen = torch.Generator().manual_seed(seed)
