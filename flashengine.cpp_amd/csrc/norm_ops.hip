@@ -328,8 +328,9 @@ __device__ __forceinline__ float silu_any(float x) { return __fdiv_rn(x, __fadd_
 // log2(e) and f the rest, taken with log2(e) in two floats.  The quotient is
 // the reciprocal estimate's, corrected once by its residual; it is subnormal
 // only for |x| < 2^-125 (bf16), where 1 + exp(-x) is 2 and quotient and
-// residual are exact.  The residual step turns a quotient of -0 into +0, so
-// the sign, which is x's everywhere, is put back.
+// residual are exact.  The residual's sign is chosen so that a quotient of -0
+// stays one: q d - x is +0 there, and -0 is added (x - q d would add +0; a
+// copysign for it took 7.42 us for 400 x 12288 in fp16 against 7.13).
 constexpr float kSiluFast = 80.f;
 __device__ __forceinline__ float silu_fast(float x) {
   constexpr float kL2e = 1.44269502162933349609375f;  // log2(e) rounded to float
@@ -340,7 +341,7 @@ __device__ __forceinline__ float silu_fast(float x) {
   const float d = __fadd_rn(1.f, e);
   const float r = __builtin_amdgcn_rcpf(d);
   const float q = __fmul_rn(x, r);
-  return __builtin_copysignf(__builtin_fmaf(__builtin_fmaf(-q, d, x), r, q), x);
+  return __builtin_fmaf(-__builtin_fmaf(q, d, -x), r, q);
 }
 
 // n / d for n < 2^31 by a multiplication: mul = floor(2^(31 + l) / d) + 1 with
