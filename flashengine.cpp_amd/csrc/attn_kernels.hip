@@ -734,9 +734,10 @@ __global__ __launch_bounds__(256, 2) void attn_tile_kernel(AttnArgs a) {
 // Per (merged row, pair of heads): lanes 0-31 take head 2hp, lanes 32-63 head
 // 2hp + 1, each lane 4 of the 128 dims, so every partial-row load is one
 // 8-byte access per lane.  Splits are folded in batches whose log-sum-exps and
-// partial rows are all in flight together.  What bounds it is that chain of round trips, not bytes:
-//   * narrow: one wavefront per pair, one batch of 4 or batches of 8, for the many rows of few
-//     splits that a full decode batch or prefill leaves.
+// partial rows are all in flight together.  What bounds it is that chain of
+// round trips, not bytes:
+//   * narrow: one wavefront per pair, one batch of 4 or batches of 8, for the
+//     many rows of few splits that a full decode batch or prefill leaves.
 //   * wide: the four wavefronts of a workgroup fold a pair's splits together,
 //     batches of 16 each, and are combined in LDS.  One sequence of 16001
 //     tokens is 128 splits, 16 round trips in the narrow form.
